@@ -71,6 +71,23 @@ struct sq_engine {
     size_t sample_cap = 0;
     void *d_passprog = nullptr;     // register-pass program of the plain sweep
     size_t passprog_cap = 0;
+    // Programs go to the device through pinned host buffers in turn, so a call
+    // neither waits for the previous call's kernels nor copies from pageable
+    // memory (16 KiB: 36 us with a stream wait and a pageable copy, 9 us so).
+    struct UploadSlot {
+        void *host = nullptr;
+        size_t cap = 0;
+        hipEvent_t copied = nullptr;   // the slot's last copy has been read
+    };
+    UploadSlot upload_slot[3];
+    int upload_next = 0;
+    // Copies `bytes` to dst on the engine's stream; src may be reused at once.
+    int upload(void *dst, const void *src, size_t bytes);
+    // Host workspaces of the plain sweep, kept between calls (their pages stay
+    // mapped; nothing in them is read by a later call).
+    std::vector<sq::LoweredGate> ws_low;
+    std::vector<unsigned char> ws_ops;
+    std::vector<int32_t> ws_key;
     void *d_scratch = nullptr;      // this device's static scratch array (sq_apply_gates_noalloc)
     int sweep_mode = 0;             // 0: register passes, 1: one launch per gate
     int pass_qbits = 5;             // register qubits per pass (1..5; set by sq_create)
@@ -139,14 +156,17 @@ struct sq_engine {
 
     int lower(const sq_gate &g, sq::LoweredGate &lg);
     int apply_lowered(const sq::LoweredGate &g);
-    int apply_plain(const std::vector<sq_gate> &gates, const std::vector<sq::LoweredGate> &low);
+    // low may be the engine's own workspace (ws_low)
+    int apply_plain(const sq_gate *gates, size_t n_gates, const std::vector<sq::LoweredGate> &low);
+    // lowers a list into ws_low; the message names the gate that fails
+    int lower_list(const sq_gate *gates, size_t n_gates);
     // CNOTs (exact U2 permutation matrices) as H CZ H when register passes run;
     // false (g2, l2 untouched) when nothing changes
-    bool expand_cnots(const std::vector<sq_gate> &gates, const std::vector<sq::LoweredGate> &low,
+    bool expand_cnots(const sq_gate *gates, const std::vector<sq::LoweredGate> &low,
                       std::vector<sq_gate> &g2, std::vector<sq::LoweredGate> &l2) const;
     // dst: where the op records go (nullptr: the engine's own growable buffer;
     // otherwise a caller-owned device buffer of dst_cap bytes, never grown)
-    int build_plain(const std::vector<sq_gate> &gates, const std::vector<sq::LoweredGate> &low, PlainProgram &prog,
+    int build_plain(const sq_gate *gates, const std::vector<sq::LoweredGate> &low, PlainProgram &prog,
                     void *dst = nullptr, size_t dst_cap = 0);
     int ensure_alt();
     // Moves index bit q of the state to bit perm[q] (a permutation of [0, n)

@@ -63,7 +63,13 @@ inline int lower_gate(const sq_gate &g, int n_qubits, LoweredGate &out, std::str
         for (int j = i + 1; j < ar; j++)
             if (g.q[i] == g.q[j]) { if (why) *why = "repeated target qubit"; return SQ_ERR_CONTRACT; }
 
-    out = LoweredGate{};
+    // m: the first four entries (all a one-qubit or diagonal gate has) cleared,
+    // a dense two-qubit gate writes all sixteen
+    out.n_pairs = 0;
+    out.diag_active = 0;
+    out.name = nullptr;
+    std::fill(out.t, out.t + 4, 0);
+    std::fill(out.m, out.m + 4, C(0.0, 0.0));
     out.k = ar;
     for (int i = 0; i < ar; i++) out.t[i] = g.q[i];
     out.pass_fraction = 1.0;

@@ -268,13 +268,9 @@ int zterms_apply(sq_engine *e, const ZTerm *d_terms, int n_terms, bool to_lambda
 // plain sweep), on psi (lambda_buffer = false) or on lambda.
 int sweep_on(sq_engine *e, const std::vector<sq_gate> &gl, bool on_lambda) {
     if (gl.empty()) return SQ_OK;
-    std::vector<LoweredGate> low(gl.size());
-    for (size_t i = 0; i < gl.size(); i++) {
-        int rc = e->lower(gl[i], low[i]);
-        if (rc) return rc;
-    }
+    if (int rc = e->lower_list(gl.data(), gl.size())) return rc;
     if (on_lambda) std::swap(e->d_state, e->d_aux);
-    const int rc = e->apply_plain(gl, low);
+    const int rc = e->apply_plain(gl.data(), gl.size(), e->ws_low);
     if (on_lambda) std::swap(e->d_state, e->d_aux);
     return rc;
 }
@@ -283,13 +279,9 @@ int sweep_on(sq_engine *e, const std::vector<sq_gate> &gl, bool on_lambda) {
 // over both vectors (twice the waves, so small states fill the GPU better).
 int sweep_both(sq_engine *e, const std::vector<sq_gate> &gl) {
     if (gl.empty()) return SQ_OK;
-    std::vector<LoweredGate> low(gl.size());
-    for (size_t i = 0; i < gl.size(); i++) {
-        int rc = e->lower(gl[i], low[i]);
-        if (rc) return rc;
-    }
+    if (int rc = e->lower_list(gl.data(), gl.size())) return rc;
     e->d_state2 = e->d_aux;
-    const int rc = e->apply_plain(gl, low);
+    const int rc = e->apply_plain(gl.data(), gl.size(), e->ws_low);
     e->d_state2 = nullptr;
     return rc;
 }

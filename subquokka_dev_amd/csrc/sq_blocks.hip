@@ -141,7 +141,7 @@ int run_blocks_mapped(sq_engine *e, const sq_gate *gates, const std::vector<Lowe
         }
         first += block_sizes[b];
     }
-    int rc = e->apply_plain(flat, flat_low);
+    int rc = e->apply_plain(flat.data(), flat.size(), flat_low);
     if (rc) return rc;
     // The reference's bit p is at bit sigma[p]: one permutation pass moves
     // every bit home (out of place, when a second copy of the state fits)
@@ -295,7 +295,7 @@ int run_blocks(sq_engine *e, const sq_gate *gates, const std::vector<LoweredGate
                 bg.push_back(gates[gi]);
                 bl.push_back(low[gi]);
             }
-            int rc = e->apply_plain(bg, bl);
+            int rc = e->apply_plain(bg.data(), bg.size(), bl);
             if (rc) return rc;
             continue;
         }

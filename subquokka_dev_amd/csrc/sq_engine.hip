@@ -259,6 +259,52 @@ int sq_engine::lower(const sq_gate &g, LoweredGate &lg) {
     return SQ_OK;
 }
 
+int sq_engine::lower_list(const sq_gate *gates, size_t n_gates) {
+    ws_low.resize(n_gates);
+    for (size_t i = 0; i < n_gates; i++)
+        if (int rc = lower(gates[i], ws_low[i])) {
+            err += " (gate " + std::to_string(i) + ")";
+            return rc;
+        }
+    return SQ_OK;
+}
+
+int sq_engine::upload(void *dst, const void *src, size_t bytes) {
+    if (!bytes) return SQ_OK;
+#if defined(__HIPCC__)
+    // A captured copy would read the slot again on replay, after other calls
+    // have written it: capture is refused, as the wait below refuses it.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipGetLastError();
+        return fail(SQ_ERR_HIP, "stream sync");
+    }
+#endif
+    UploadSlot &s = upload_slot[upload_next];
+    upload_next = (upload_next + 1) % 3;
+    hipError_t he = hipSuccess;
+    if (!s.copied) {
+        he = hipEventCreate(&s.copied);
+        if (he != hipSuccess) return hip_fail(he, "hipEventCreate(upload)");
+    } else if ((he = hipEventSynchronize(s.copied)) != hipSuccess) {
+        return hip_fail(he, "stream sync");
+    }
+    if (bytes > s.cap) {
+        if (s.host) hipHostFree(s.host);
+        s.host = nullptr;
+        s.cap = 0;
+        const size_t want = std::max<size_t>(bytes * 2, 65536);
+        he = hipHostMalloc(&s.host, want, hipHostMallocDefault);
+        if (he != hipSuccess) return hip_fail(he, "hipHostMalloc(upload)");
+        s.cap = want;
+    }
+    std::memcpy(s.host, src, bytes);
+    he = hipMemcpyAsync(dst, s.host, bytes, hipMemcpyHostToDevice, stream);
+    if (he == hipSuccess) he = hipEventRecord(s.copied, stream);
+    return he == hipSuccess ? SQ_OK : hip_fail(he, "hipMemcpyAsync(upload)");
+}
+
 // ---------------------------------------------------------------------------
 // reductions (partials summed on the host in block order)
 // ---------------------------------------------------------------------------
@@ -378,6 +424,10 @@ int sq_destroy(sq_engine *e) {
     if (e->d_alt) hipFree(e->d_alt);
     if (e->d_part) hipFree(e->d_part);
     if (e->d_stage) hipFree(e->d_stage);
+    for (auto &u : e->upload_slot) {
+        if (u.copied) hipEventDestroy(u.copied);
+        if (u.host) hipHostFree(u.host);
+    }
     e->free_extras();
     if (e->stream) hipStreamDestroy(e->stream);
     delete e;
@@ -474,13 +524,9 @@ int sq_apply_gates(sq_engine *e, const sq_gate *gates, uint64_t n) {
     if (!e || (!gates && n)) return SQ_ERR_ARG;
     SQ_HIP(hipSetDevice(e->device));
     // Validate everything first so a bad line leaves the state untouched.
-    std::vector<LoweredGate> low(n);
-    for (uint64_t i = 0; i < n; i++) {
-        int rc = e->lower(gates[i], low[i]);
-        if (rc) { e->err += " (gate " + std::to_string(i) + ")"; return rc; }
-    }
-    if (e->out_of_core()) return e->stream_apply(std::vector<sq_gate>(gates, gates + n), low);
-    return e->apply_plain(std::vector<sq_gate>(gates, gates + n), low);
+    if (int rc = e->lower_list(gates, n)) return rc;
+    if (e->out_of_core()) return e->stream_apply(std::vector<sq_gate>(gates, gates + n), e->ws_low);
+    return e->apply_plain(gates, n, e->ws_low);
 }
 
 int sq_norm2(sq_engine *e, double *out) {

@@ -37,8 +37,60 @@ namespace {
 static_assert(kPassMaxKH <= 5, "PlainLaunch holds five register qubits");
 static_assert(kPassLaneHi == 3, "PlainLaunch holds three lane positions");
 
+// The op records of a program, in a byte workspace that outlives the call.
+template <typename T> class OpBuffer {
+    std::vector<unsigned char> &mem;
+    size_t n = 0;
+
+public:
+    explicit OpBuffer(std::vector<unsigned char> &m) : mem(m) {}
+    PassOp<T> *extend(size_t k) {   // k more records (contents undefined)
+        const size_t need = (n + k) * sizeof(PassOp<T>) + alignof(PassOp<T>);
+        if (need > mem.size()) {
+            // keep the records where alignment puts them in the larger block
+            std::vector<unsigned char> next(std::max(need, 2 * mem.size()));
+            std::swap(mem, next);
+            if (n) std::memcpy(static_cast<void *>(data()), align(next), n * sizeof(PassOp<T>));
+        }
+        n += k;
+        return data() + (n - k);
+    }
+    void push_back(const PassOp<T> &o) { *extend(1) = o; }
+    PassOp<T> *data() { return static_cast<PassOp<T> *>(align(mem)); }
+    PassOp<T> &operator[](size_t i) { return data()[i]; }
+    PassOp<T> &back() { return data()[n - 1]; }
+    size_t size() const { return n; }
+    bool empty() const { return n == 0; }
+
+private:
+    static void *align(std::vector<unsigned char> &m) {
+        const uintptr_t a = alignof(PassOp<T>);
+        return reinterpret_cast<void *>((reinterpret_cast<uintptr_t>(m.data()) + a - 1) / a * a);
+    }
+};
+
+// A gate of a register pass: dense on one qubit or diagonal on one or two, in
+// the pass's virtual positions (t ascending).
+struct PassGate {
+    OpClass cls;
+    int k;
+    int t[2];
+    std::complex<double> m[4];
+    uint32_t diag_active;
+    // the lowered gate with its targets mapped through vpos (sq::relabel)
+    PassGate(const LoweredGate &g, const std::vector<int> &vpos)
+        : cls(g.cls), k(g.k), t{vpos[g.t[0]], g.k > 1 ? vpos[g.t[1]] : 0}, m{g.m[0], g.m[1], g.m[2], g.m[3]},
+          diag_active(g.diag_active) {
+        if (k == 2 && t[0] > t[1]) {
+            std::swap(t[0], t[1]);
+            std::swap(m[1], m[2]);
+            diag_active = (diag_active & 9u) | ((diag_active & 2u) << 1) | ((diag_active & 4u) >> 1);
+        }
+    }
+};
+
 template <typename T>
-void encode_pass_op(const LoweredGate &g, const std::vector<int> &regs, std::vector<PassOp<T>> &ops) {
+void encode_pass_op(const PassGate &g, const std::vector<int> &regs, OpBuffer<T> &ops) {
     constexpr int VB = Traits<T>::VB;
     constexpr int S = VB + 6;
     auto slot = [&](int t) {
@@ -165,7 +217,7 @@ struct PhaseSplit {
     std::complex<double> g{1.0, 0.0}, zl{1.0, 0.0}, zr{1.0, 0.0};
     double c = 1.0, s = 0.0;
 };
-PhaseSplit phase_split(const LoweredGate &u) {
+PhaseSplit phase_split(const PassGate &u) {
     PhaseSplit p;
     if (u.cls != OpClass::Dense || u.k != 1) return p;
     bool real = true;
@@ -231,11 +283,11 @@ PassOp<T> rotation_op(double c, double s, int q, const std::vector<int> &regs, d
 // CP(pi) / CZ as lowered: a two-qubit diagonal whose only entry other than 1
 // is -1 (within one ulp: e^{i pi} evaluates to -1 + 1.2e-16 i; leaving out
 // that term changes each amplitude by less than one ulp of its magnitude).
-bool is_sign_cp(const LoweredGate &d) {
+bool is_sign_cp(const PassGate &d) {
     return d.cls == OpClass::Diag && d.k == 2 && d.diag_active == 8u && d.m[3].real() == -1.0 &&
            std::abs(d.m[3].imag()) <= 0x1p-52;
 }
-template <typename T> PassOp<T> sign_op(const LoweredGate &d, const std::vector<int> &regs, int S) {
+template <typename T> PassOp<T> sign_op(const PassGate &d, const std::vector<int> &regs, int S) {
     PassOp<T> o{};
     o.kind = PO_SIGN;
     o.pad[0] = o.pad[1] = -1;
@@ -256,8 +308,8 @@ template <typename T> PassOp<T> sign_op(const LoweredGate &d, const std::vector<
 // own (half the registers), two or more into the 2^KH table.  Returns the FP
 // operations per amplitude.
 template <typename T>
-double emit_phases(const std::vector<std::complex<double>> &fac, const std::vector<int> &regs, int S,
-                   std::complex<double> gs, std::vector<PassOp<T>> &ops) {
+double emit_phases(const std::complex<double> *fac, const std::vector<int> &regs, int S,
+                   std::complex<double> gs, OpBuffer<T> &ops) {
     static_assert(sizeof(PassOp<T>) == 8 * sizeof(cx<T>), "a coefficient record holds 8 coefficients");
     const std::complex<double> one(1.0, 0.0);
     int lane_mask = 0;
@@ -326,7 +378,7 @@ int launch_pass(sq_engine *e, const PassArgs<T> &a) {
 }
 
 template <typename T>
-int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::vector<LoweredGate> &low,
+int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredGate> &low,
                   PlainProgram &prog, void *dst, size_t dst_cap) {
     constexpr int VB = Traits<T>::VB;
     constexpr int S = VB + 6;
@@ -339,7 +391,7 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         prog.per_gate = true;
         return SQ_OK;
     }
-    const size_t ng = gates.size();
+    const size_t ng = low.size();
     std::vector<char> mergeable(ng, 0), anywhere(ng, 0);
     for (size_t i = 0; i < ng; i++) {
         const LoweredGate &g = low[i];
@@ -352,8 +404,9 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
     // The schedule depends on the gates' qubits and classes only: a list
     // with the structure of a recent one (the same circuit again, or with new
     // angles) reuses its schedule; the op records are encoded every call.
-    std::vector<int32_t> key = {n, S, kh, moves, std::min(n - 1, 27 + VB), e->plan_beam, (int32_t)ng};
-    key.reserve(6 + 6 * ng);
+    std::vector<int32_t> &key = e->ws_key;
+    key.assign({n, S, kh, moves, std::min(n - 1, 27 + VB), e->plan_beam, (int32_t)ng});
+    key.reserve(7 + 5 * ng);
     for (size_t i = 0; i < ng; i++) {
         key.push_back(mergeable[i] | (anywhere[i] << 1) | (gates[i].nq << 2));
         for (int j = 0; j < gates[i].nq && j < 4; j++) key.push_back(gates[i].q[j]);
@@ -367,16 +420,20 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
     }
     if (!steps_ptr) {
         sq_engine::PlanCacheEntry ent;
-        ent.steps = sq::plan_register_passes(gates, mergeable, anywhere, n, S, kh, moves, std::min(n - 1, 27 + VB),
+        ent.steps = sq::plan_register_passes(std::vector<sq_gate>(gates, gates + ng), mergeable, anywhere, n, S, kh, moves, std::min(n - 1, 27 + VB),
                                              e->plan_beam);
-        ent.key = std::move(key);
+        ent.key = key;
         e->plan_cache.insert(e->plan_cache.begin(), std::move(ent));
         if (e->plan_cache.size() > 4) e->plan_cache.pop_back();
         steps_ptr = &e->plan_cache[0].steps;
     }
     const std::vector<sq::SweepStep> &steps = *steps_ptr;
 
-    std::vector<PassOp<T>> ops;
+    OpBuffer<T> ops(e->ws_ops);
+    std::vector<PassGate> lg;
+    std::vector<PhaseSplit> sp;
+    std::vector<int> fold_into, folded_from, next;
+    std::vector<char> absorbed, zr_done;
     for (const auto &st : steps) {
         double frac = 0;
         for (int gi : st.gates) frac += low[gi].pass_fraction;
@@ -409,14 +466,21 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         std::sort(regs.begin(), regs.end());
         l.merged = true;
         l.op_begin = (int)ops.size();
-        std::vector<LoweredGate> lg;
-        lg.reserve(st.gates.size());
-        for (int gi : st.gates) {
-            lg.push_back(low[gi]);
-            sq::relabel(lg.back(), vpos);
-        }
+        lg.clear();
+        for (int gi : st.gates) lg.emplace_back(low[gi], vpos);
+        // next[2 i + x]: the next gate on gate i's x-th target; head[q]: the
+        // first one on q (kept at or after the gate being encoded)
+        const int N = (int)lg.size();
+        std::vector<int> head(n, N);
+        next.assign(2 * N, N);
+        for (int i = N; i-- > 0;)
+            for (int x = 0; x < lg[i].k; x++) {
+                next[2 * i + x] = head[lg[i].t[x]];
+                head[lg[i].t[x]] = i;
+            }
+        auto next_on = [&](int i, int q) { return next[2 * i + (lg[i].t[0] == q ? 0 : 1)]; };
         const std::complex<double> one(1.0, 0.0);
-        std::vector<PhaseSplit> sp(lg.size());
+        sp.assign(N, PhaseSplit{});
         bool any_split = false;
         if (e->phase_split)
             for (size_t i = 0; i < lg.size(); i++) {
@@ -427,23 +491,20 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         // next gate on either qubit is a dense gate on a register slot or a
         // lane bit goes into that gate's op, with the other qubit as the control
         // (not into a split gate: its rotation runs as shears)
-        std::vector<int> fold_into(lg.size(), -1), folded_from(lg.size(), -1);
+        fold_into.assign(N, -1);
+        folded_from.assign(N, -1);
         if constexpr (sizeof(T) == 8) {
             auto in_regs = [&](int t) { return std::find(regs.begin(), regs.end(), t) != regs.end(); };
             for (size_t i = 0; i < lg.size(); i++) {
-                const LoweredGate &d = lg[i];
+                const PassGate &d = lg[i];
                 if (!(d.cls == OpClass::Diag && d.k == 2 && d.diag_active == 8u)) continue;
-                for (size_t j = i + 1; j < lg.size(); j++) {
-                    const LoweredGate &u = lg[j];
-                    bool touches = false;
-                    for (int x = 0; x < u.k; x++) touches = touches || u.t[x] == d.t[0] || u.t[x] == d.t[1];
-                    if (!touches) continue;
-                    if (u.cls == OpClass::Dense && u.k == 1 && folded_from[j] < 0 && !sp[j].ok &&
-                        (in_regs(u.t[0]) || (u.t[0] >= VB && u.t[0] < S))) {
-                        fold_into[i] = (int)j;
-                        folded_from[j] = (int)i;
-                    }
-                    break;
+                const int j = std::min(next[2 * i], next[2 * i + 1]);   // the next gate on either qubit
+                if (j == N) continue;
+                const PassGate &u = lg[j];
+                if (u.cls == OpClass::Dense && folded_from[j] < 0 && !sp[j].ok &&
+                    (in_regs(u.t[0]) || (u.t[0] >= VB && u.t[0] < S))) {
+                    fold_into[i] = j;
+                    folded_from[j] = (int)i;
                 }
             }
         }
@@ -456,28 +517,30 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         // gpass; the pass ends with a flush of what is left.
         auto resident = [&](int t) { return t < S || std::find(regs.begin(), regs.end(), t) != regs.end(); };
         std::vector<std::complex<double>> pend(n, one);
-        std::vector<char> absorbed(lg.size(), 0), zr_done(lg.size(), 0);
+        absorbed.assign(N, 0);
+        zr_done.assign(N, 0);
         std::complex<double> gpass = one;
         auto diag1 = [&](size_t j) {
-            const LoweredGate &d = lg[j];
+            const PassGate &d = lg[j];
             return any_split && d.cls == OpClass::Diag && d.k == 1 && resident(d.t[0]) && d.m[0] != 0.0;
         };
-        auto flush = [&](size_t from, bool last) {
-            std::vector<std::complex<double>> fac(n, one);
+        auto flush = [&](int from, bool last) {
+            std::complex<double> fac[64];
             auto take = [&](int q) {
                 std::complex<double> f = pend[q];
                 pend[q] = one;
-                for (size_t j = from; j < lg.size(); j++) {
-                    const LoweredGate &u = lg[j];
+                int &h = head[q];
+                while (h < from) h = next_on(h, q);
+                for (int j = h; j < N; j = next_on(j, q)) {
+                    const PassGate &u = lg[j];
                     if (u.cls == OpClass::Diag) {
-                        if (diag1(j) && u.t[0] == q && !absorbed[j]) {
+                        if (diag1(j) && !absorbed[j]) {
                             f *= u.m[1] / u.m[0];
                             gpass *= u.m[0];
                             absorbed[j] = 1;
                         }
                         continue;
                     }
-                    if (u.t[0] != q) continue;
                     if (sp[j].ok && !zr_done[j]) {
                         f *= sp[j].zr;
                         zr_done[j] = 1;
@@ -509,7 +572,7 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
                 ops.push_back(sign_op<T>(lg[i], regs, S));
                 continue;
             }
-            LoweredGate gi = lg[i];
+            PassGate gi = lg[i];
             if (any_split && gi.cls == OpClass::Dense) {
                 const int q = gi.t[0];
                 std::complex<double> need = pend[q];
@@ -539,7 +602,7 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
             }
             encode_pass_op<T>(gi, regs, ops);
             if constexpr (sizeof(T) == 8) if (folded_from[i] >= 0) {
-                const LoweredGate &d = lg[folded_from[i]];
+                const PassGate &d = lg[folded_from[i]];
                 PassOp<T> &o = ops.back();
                 const int ctl = gi.t[0] == d.t[0] ? d.t[1] : d.t[0];
                 const auto it = std::find(regs.begin(), regs.end(), ctl);
@@ -593,7 +656,7 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         if (idx >= 0) e->pass_census[idx]++;
     }
 
-    // upload the program once; earlier launches may still read the old one
+    // upload the program once (in stream order: earlier launches may still read the old one)
     const size_t need = ops.size() * sizeof(PassOp<T>) + 256;
     if (dst) {   // caller-owned buffer: never grown
         if (ops.size() * sizeof(PassOp<T>) > dst_cap)
@@ -608,8 +671,8 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
         return SQ_OK;
     }
     if (!ops.empty()) {
-        if (hipStreamSynchronize(e->stream) != hipSuccess) return e->fail(SQ_ERR_HIP, "stream sync");
         if (need > e->passprog_cap) {
+            if (hipStreamSynchronize(e->stream) != hipSuccess) return e->fail(SQ_ERR_HIP, "stream sync");
             if (e->d_passprog) (void)hipFree(e->d_passprog);
             e->d_passprog = nullptr;
             e->passprog_cap = 0;
@@ -617,9 +680,7 @@ int build_plain_t(sq_engine *e, const std::vector<sq_gate> &gates, const std::ve
             if (he != hipSuccess) return e->hip_fail(he, "hipMalloc(pass program)");
             e->passprog_cap = need * 2;
         }
-        char *d = static_cast<char *>(e->d_passprog);
-        hipError_t he = hipMemcpy(d, ops.data(), ops.size() * sizeof(PassOp<T>), hipMemcpyHostToDevice);
-        if (he != hipSuccess) return e->hip_fail(he, "hipMemcpy(pass program)");
+        if (int rc = e->upload(e->d_passprog, ops.data(), ops.size() * sizeof(PassOp<T>))) return rc;
     }
     prog.d_ops = e->d_passprog;
     return SQ_OK;
@@ -702,7 +763,7 @@ int run_plain_t(sq_engine *e, const PlainProgram &prog, const std::vector<Lowere
 
 }  // namespace
 
-int sq_engine::build_plain(const std::vector<sq_gate> &gates, const std::vector<LoweredGate> &low, PlainProgram &prog,
+int sq_engine::build_plain(const sq_gate *gates, const std::vector<LoweredGate> &low, PlainProgram &prog,
                            void *dst, size_t dst_cap) {
     return dtype == SQ_C128 ? build_plain_t<double>(this, gates, low, prog, dst, dst_cap)
                             : build_plain_t<float>(this, gates, low, prog, dst, dst_cap);
@@ -756,7 +817,7 @@ int cnot_target(const LoweredGate &g) {
 // coefficients, so it joins a pass (on complex128 the CZ folds into the
 // second H) instead of taking a pass of its own.  The products differ from
 // the dense 4x4 application by rounding only (|H H - I| = 2^-52).
-bool sq_engine::expand_cnots(const std::vector<sq_gate> &gates, const std::vector<LoweredGate> &low,
+bool sq_engine::expand_cnots(const sq_gate *gates, const std::vector<LoweredGate> &low,
                              std::vector<sq_gate> &g2, std::vector<LoweredGate> &l2) const {
     const int S = (dtype == SQ_C64 ? 1 : 0) + 6;
     if (sweep_mode != 0 || n < S + pass_qbits) return false;   // no register passes
@@ -804,12 +865,13 @@ bool sq_engine::expand_cnots(const std::vector<sq_gate> &gates, const std::vecto
     return true;
 }
 
-int sq_engine::apply_plain(const std::vector<sq_gate> &gates, const std::vector<LoweredGate> &low) {
+int sq_engine::apply_plain(const sq_gate *gates, size_t n_gates, const std::vector<LoweredGate> &low) {
+    if (low.size() != n_gates) return fail(SQ_ERR_ARG, "internal: lowered list of another size");
     std::vector<sq_gate> g2;
     std::vector<LoweredGate> l2;
     const bool x = expand_cnots(gates, low, g2, l2);
     PlainProgram prog;
-    int rc = build_plain(x ? g2 : gates, x ? l2 : low, prog);
+    int rc = build_plain(x ? g2.data() : gates, x ? l2 : low, prog);
     return rc ? rc : run_plain_program(prog, x ? l2 : low);
 }
 
@@ -856,18 +918,13 @@ extern "C" int sq_apply_gates_noalloc(sq_engine *e, const sq_gate *gates, uint64
     if (hipSetDevice(e->device) != hipSuccess) return e->fail(SQ_ERR_HIP, "hipSetDevice");
     // validate everything first so a bad line (or a program too large for the
     // scratch) leaves the state untouched
-    std::vector<LoweredGate> low(n);
-    for (uint64_t i = 0; i < n; i++) {
-        int rc = e->lower(gates[i], low[i]);
-        if (rc) { e->err += " (gate " + std::to_string(i) + ")"; return rc; }
-    }
-    const std::vector<sq_gate> gl(gates, gates + n);
+    if (int rc = e->lower_list(gates, n)) return rc;
     std::vector<sq_gate> g2;
     std::vector<LoweredGate> l2;
-    const bool x = e->expand_cnots(gl, low, g2, l2);
+    const bool x = e->expand_cnots(gates, e->ws_low, g2, l2);
     PlainProgram prog;
-    int rc = e->build_plain(x ? g2 : gl, x ? l2 : low, prog, e->d_scratch, kScratchBytes);
-    return rc ? rc : e->run_plain_program(prog, x ? l2 : low);
+    int rc = e->build_plain(x ? g2.data() : gates, x ? l2 : e->ws_low, prog, e->d_scratch, kScratchBytes);
+    return rc ? rc : e->run_plain_program(prog, x ? l2 : e->ws_low);
 }
 
 extern "C" int sq_pass_census(sq_engine *e, int64_t *counts, int32_t cap, int32_t *n_out) {

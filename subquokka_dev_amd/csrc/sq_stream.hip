@@ -449,7 +449,7 @@ int sq_engine::stream_apply(const std::vector<sq_gate> &gates, const std::vector
         // uploaded once, run on every group
         PlainProgram prog;
         n = W;
-        rc = build_plain(pgates, pg, prog);
+        rc = build_plain(pgates.data(), pg, prog);
         n = saved_n;
         if (rc) break;
         std::vector<uint64_t> run_off(1ULL << h), run_off_bytes(1ULL << h);   // host offset of run r within a group
