@@ -68,6 +68,16 @@ enum PassOpKind : int32_t {
     PO_SIGN = 11,        // amplitude i negated where every bit of i named below is 1 (CP(pi),
                          //   CZ): a = mask of virtual positions < VB + 6, b = mask of register
                          //   slots, pad[0], pad[1] = tile positions (-1: none)
+    PO_DIAG_TAB = 12,    // a run of diagonal gates in one product: amplitude i times F(i) when
+                         //   bit a of its register index is 1 (a < 0: every amplitude), F from
+                         //   complex<double> tables in the c records after the op:
+                         //     64 << VB entries by lane and vector element;
+                         //     per tile-number bit of `active` (ascending), applied when set:
+                         //       a >= 0: one entry;  a < 0: 64 << VB entries by lane and element;
+                         //     b = 1 (a < 0 only): rows of 32 entries by tile-number bit q --
+                         //       the first, then one per bit p of pad[0] (ascending, applied when
+                         //       p is set) -- whose products over the rows are multiplied over
+                         //       the set bits q.
 };
 // Dense ops (PO_DENSE_REG/_C, PO_DENSE_LANE/_C, PO_DENSE_VEC) with c = 15 have
 // four real coefficients (after a fold, also the folded ones): the kernel
@@ -673,6 +683,45 @@ __device__ inline void pass_diag_reg2(Pack<T> (&v)[R], const Coef4<T> d, uint32_
     }
 }
 
+// PO_DIAG_TAB's factor of one lane and vector element.  One gate costs a pass
+// four FP64 products per register it touches; here the gates that share a
+// register slot (or none) first meet in one factor per lane -- a table entry
+// for the lane bits, one product per set tile bit -- and the registers are
+// multiplied once.  Five layers of RZZ on the complete graph of 21 qubits
+// (complex128, 13 passes): 475 -> 199 us.
+template <int E> struct DiagTab {
+    const cx<double> *lane_rows;   // 64 E entries per row
+    int lane;
+    __device__ cx<double> at(int row, int e) const { return lane_rows[(row * 64 + lane) * E + e]; }
+};
+// Entry j of a table read by the whole wave (scalar loads).
+__device__ inline cx<double> diag_tab_uniform(const cx<double> *t, int j) {
+    typedef SQK_AS_CONST const double cpd;
+    cpd *q = (cpd *)(t + j);
+    return {q[0], q[1]};
+}
+// The product over tile-number bits (PO_DIAG_TAB, b = 1): lane q holds bit q's
+// row product; the set bits' products are multiplied across the lanes.
+__device__ inline cx<double> diag_tab_tiles(const cx<double> *rows, uint32_t mask, uint32_t t, int lane) {
+    auto of_bit = [&](int q) {
+        cx<double> g = rows[q];
+        const cx<double> *row = rows + 32;
+        for (uint32_t m = mask; m; m &= m - 1, row += 32)
+            if ((t >> __builtin_ctz(m)) & 1) g = cmul(g, row[q]);
+        return (t >> q) & 1 ? g : cx<double>{1.0, 0.0};
+    };
+#if defined(__HIP_DEVICE_COMPILE__)
+    cx<double> g = of_bit(lane & 31);
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) g = cmul(g, cx<double>{__shfl_xor(g.re, o, 64), __shfl_xor(g.im, o, 64)});
+#else
+    (void)lane;
+    cx<double> g = of_bit(0);   // the host build runs one lane at a time
+    for (int q = 1; q < 32; q++) g = cmul(g, of_bit(q));
+#endif
+    return g;
+}
+
 template <typename T, int R, int E, bool SU, int RM>
 __device__ inline void pass_dense_lane_at(Pack<T> (&v)[R], int a, bool hi, const Coef4<T> k) {
     switch (a) {
@@ -856,6 +905,50 @@ __global__ void __launch_bounds__(kBlock) k_pass(cx<T> *__restrict__ s, const Pa
                     if ((r & o.b) == o.b)
 #pragma unroll
                         for (int e = 0; e < E; e++) flip_sign(v[r].e[e], mk[e]);
+                break; }
+            case PO_DIAG_TAB: {
+                const DiagTab<E> tab{reinterpret_cast<const cx<double> *>(a.ops + op + 1), lane};
+                cx<double> f[E];
+#pragma unroll
+                for (int e = 0; e < E; e++) f[e] = tab.at(0, e);
+                const cx<double> *rest = tab.lane_rows + 64 * E;
+                const uint32_t tn = (uint32_t)t;   // at most kPassMaxTileBits bits
+                if (o.a < 0) {
+                    int row = 1;
+                    for (uint32_t m = o.active; m; m &= m - 1, row++)
+                        if ((tn >> __builtin_ctz(m)) & 1)
+#pragma unroll
+                            for (int e = 0; e < E; e++) f[e] = cmul(f[e], tab.at(row, e));
+                    if (o.b) {
+                        const cx<double> g = diag_tab_tiles(tab.lane_rows + row * 64 * E, (uint32_t)rec.dw(5), tn, lane);
+#pragma unroll
+                        for (int e = 0; e < E; e++) f[e] = cmul(f[e], g);
+                    }
+                } else {
+                    cx<double> g = {1.0, 0.0};
+                    int j = 0;
+                    for (uint32_t m = o.active; m; m &= m - 1, j++)
+                        if ((tn >> __builtin_ctz(m)) & 1) g = cmul(g, diag_tab_uniform(rest, j));
+#pragma unroll
+                    for (int e = 0; e < E; e++) f[e] = cmul(f[e], g);
+                }
+                cx<T> ft[E];
+#pragma unroll
+                for (int e = 0; e < E; e++) ft[e] = {(T)f[e].re, (T)f[e].im};
+                switch (o.a) {
+                case 0: pass_diag_reg1<T, 0, R, E>(v, ft, ft, false, true); break;
+                case 1: if constexpr (KH > 1) pass_diag_reg1<T, 1, R, E>(v, ft, ft, false, true); break;
+                case 2: if constexpr (KH > 2) pass_diag_reg1<T, 2, R, E>(v, ft, ft, false, true); break;
+                case 3: if constexpr (KH > 3) pass_diag_reg1<T, 3, R, E>(v, ft, ft, false, true); break;
+                case 4: if constexpr (KH > 4) pass_diag_reg1<T, 4, R, E>(v, ft, ft, false, true); break;
+                default:
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+#pragma unroll
+                        for (int e = 0; e < E; e++) ip_cmul(v[r].e[e], ft[e]);
+                    break;
+                }
+                op += o.c;   // past the tables
                 break; }
             case PO_PHASES: {
                 // L per lane (and vector element): the scalar times z_p for each

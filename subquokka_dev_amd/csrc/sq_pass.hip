@@ -366,6 +366,314 @@ double emit_phases(const std::complex<double> *fac, const std::vector<int> &regs
     return flops;
 }
 
+// Runs of diagonal gates (PO_DIAG_TAB).  A diagonal gate with entries of
+// modulus 1 is a scalar, a phase per qubit and a controlled phase:
+//   diag(d0, d1, d2, d3) = d0 diag(1, z0)(t0) diag(1, z1)(t1) diag(1, 1, 1, c)(t0 t1).
+// The factors of a run are collected in long double: gates of a layer often
+// share their angle, and the rounding of a quotient would then add up over
+// them instead of averaging out (21-qubit MaxCut layers, error against 64
+// bits: 7e-14 with double factors, 5e-15 as here and as with one op per gate).
+struct Ext {
+    long double re = 1.0L, im = 0.0L;
+    Ext() = default;
+    Ext(const std::complex<double> &z) : re(z.real()), im(z.imag()) {}
+    Ext(long double r, long double i) : re(r), im(i) {}
+    bool one() const { return re == 1.0L && im == 0.0L; }
+    Ext operator*(const Ext &o) const { return {re * o.re - im * o.im, re * o.im + im * o.re}; }
+    // 1 / z for |z|^2 = 1 + e, |e| <= 1e-9: conj(z) (1 - e + e^2)
+    Ext inv() const {
+        const long double e = (re * re - 1.0L) + im * im, s = 1.0L - e + e * e;
+        return {re * s, -im * s};
+    }
+    std::complex<double> hi() const { return {(double)re, (double)im}; }
+    std::complex<double> lo() const { return {(double)(re - (double)re), (double)(im - (double)im)}; }
+};
+bool unit_diagonal(const PassGate &d) {
+    for (int i = 0; i < (1 << d.k); i++)
+        if (!(std::abs(d.m[i].real() * d.m[i].real() + d.m[i].imag() * d.m[i].imag() - 1.0) <= 1e-9)) return false;
+    return true;
+}
+
+// Where a pass's virtual positions lie.
+struct PassMap {
+    enum { Lane = 0, Slot = 1, Tile = 2 };
+    int S = 0, n = 0, n_regs = 0, n_tile = 0;
+    PassMap() = default;
+    char kind[64];
+    char idx[64];        // lane position / register slot / tile-number bit
+    int slot_pos[8];
+    PassMap(int S_, int n_, const std::vector<int> &regs) : S(S_), n(n_), n_regs((int)regs.size()) {
+        for (int p = 0; p < n; p++) { kind[p] = p < S ? Lane : Tile; idx[p] = (char)p; }
+        for (int j = 0; j < n_regs; j++) { kind[regs[j]] = Slot; idx[regs[j]] = (char)j; slot_pos[j] = regs[j]; }
+        for (int p = S; p < n; p++) if (kind[p] == Tile) idx[p] = (char)n_tile++;
+    }
+};
+
+// Diagonal gates of a pass that wait for the next dense gate on one of their
+// qubits (they commute with each other and with everything on other qubits),
+// in virtual positions.
+template <typename T> struct DiagRun {
+    static constexpr int VB = Traits<T>::VB, S = VB + 6, NL = 64 << VB;
+    using C = std::complex<double>;
+    PassMap map;
+    std::vector<const PassGate *> gates;
+    uint64_t touched = 0;    // positions of the gates
+    // which factors the run has: by slot its lane and tile partners, by lane
+    // position its higher lane partners, by tile bit its lane and higher tile
+    // partners; pairs of slots (bit 8 j + k, j < k); positions with a phase
+    uint32_t slot_lane[8] = {}, slot_tile[8] = {}, lane_lane[8] = {}, tile_lane[32] = {}, tile_tile[32] = {};
+    uint64_t slot_slot = 0, single = 0;
+    bool scalar = false;
+    double old_cost = 0;     // one op per gate (unit: all registers times one factor per lane)
+    explicit DiagRun(int n) : z(n), pair((size_t)n * n) {}
+    void start(const std::vector<int> &regs) { map = PassMap(S, (int)z.size(), regs); }
+    void clear() {
+        gates.clear();
+        touched = slot_slot = single = 0;
+        for (uint32_t *a : {slot_lane, slot_tile, lane_lane}) std::fill(a, a + 8, 0u);
+        std::fill(tile_lane, tile_lane + 32, 0u);
+        std::fill(tile_tile, tile_tile + 32, 0u);
+        scalar = false;
+        old_cost = 0;
+    }
+
+    void add(const PassGate &d) {
+        gates.push_back(&d);
+        const C one(1.0, 0.0);
+        scalar = scalar || d.m[0] != one;
+        const int a = d.t[0], ka = map.kind[a], ia = map.idx[a];
+        const uint32_t act = d.diag_active;
+        touched |= 1ULL << a;
+        if (d.m[1] != d.m[0]) single |= 1ULL << a;
+        if (d.k == 1) {
+            old_cost += 0.15 + (ka == PassMap::Lane ? 1.0 : 0.5 * __builtin_popcount(act & 3u));
+            return;
+        }
+        const int b = d.t[1], kb = map.kind[b], ib = map.idx[b];
+        touched |= 1ULL << b;
+        if (d.m[2] != d.m[0]) single |= 1ULL << b;
+        const double quarter = 0.15 + __builtin_popcount(act & 15u) / 4.0;
+        if (ka == PassMap::Slot && kb == PassMap::Slot) {
+            slot_slot |= 1ULL << (8 * std::min(ia, ib) + std::max(ia, ib));
+            old_cost += quarter;
+        } else if (ka == PassMap::Slot || kb == PassMap::Slot) {
+            const int j = ka == PassMap::Slot ? ia : ib, ko = ka == PassMap::Slot ? kb : ka, io = ka == PassMap::Slot ? ib : ia;
+            (ko == PassMap::Lane ? slot_lane : slot_tile)[j] |= 1u << io;
+            const uint32_t half0 = ka == PassMap::Slot ? 5u : 3u;   // entries whose slot bit is 0
+            old_cost += ko == PassMap::Tile ? quarter : 0.15 + 0.5 * (((act & half0) != 0) + ((act & ~half0 & 15u) != 0));
+        } else if (ka == PassMap::Tile && kb == PassMap::Tile) {
+            tile_tile[std::min(ia, ib)] |= 1u << std::max(ia, ib);
+            old_cost += quarter;
+        } else {
+            if (ka == PassMap::Lane && kb == PassMap::Lane) lane_lane[std::min(ia, ib)] |= 1u << std::max(ia, ib);
+            else tile_lane[ka == PassMap::Tile ? ia : ib] |= 1u << (ka == PassMap::Tile ? ib : ia);
+            old_cost += 1.15;
+        }
+    }
+    bool slot_table(int j) const { return slot_lane[j] || slot_tile[j]; }
+    bool tile_singles() const { return (single & ~slot_positions()) >> S; }
+    uint64_t slot_positions() const {
+        uint64_t m = 0;
+        for (int j = 0; j < map.n_regs; j++) m |= 1ULL << map.slot_pos[j];
+        return m;
+    }
+    bool has_tiles() const {
+        for (int k = 0; k < map.n_tile; k++) if (tile_tile[k]) return true;
+        return tile_singles();
+    }
+    bool has_all() const {
+        if (scalar || (single & ((1ULL << S) - 1)) || has_tiles()) return true;
+        for (int p = 0; p < S; p++) if (lane_lane[p]) return true;
+        for (int k = 0; k < map.n_tile; k++) if (tile_lane[k]) return true;
+        return false;
+    }
+    // The run as tables, in the unit of old_cost: 0.05 / 0.03 per tile bit's
+    // row of lane entries / one entry (half of them are applied), 0.5 + 0.08
+    // per row for the products over tile bits.  With fewer than three waves
+    // per SIMD nothing hides a table's fetch (about 500 cycles, one
+    // multiplication of 32 registers): `late` adds it.
+    double cost() const {
+        const double late = map.n_tile < 12 ? 1.0 : 0.0;
+        double c = 0;
+        if (has_all()) {
+            c += 1.2 + late;
+            for (int k = 0; k < map.n_tile; k++) c += (tile_lane[k] ? 0.05 : 0.0) + (tile_tile[k] ? 0.08 : 0.0);
+            if (has_tiles()) c += 0.5 + late;
+        }
+        for (int j = 0; j < map.n_regs; j++) {
+            if (slot_table(j)) c += 0.7 + late + 0.03 * __builtin_popcount(slot_tile[j]);
+            else if ((single >> map.slot_pos[j]) & 1) c += 0.65;
+        }
+        return c + 0.4 * __builtin_popcountll(slot_slot);
+    }
+
+    // Appends the run as ops; due[p]: further phases of position p (below S or
+    // a slot), may be null.  Returns the FP operations per amplitude.
+    double emit(OpBuffer<T> &ops, const C *due) {
+        const double flops = emit_tables(ops, due);
+        std::fill(z.begin(), z.end(), Ext());
+        for (const PassGate *d : gates)
+            if (d->k == 2) pair[std::min(d->t[0], d->t[1]) * map.n + std::max(d->t[0], d->t[1])] = Ext();
+        return flops;
+    }
+
+private:
+    std::vector<Ext> z, pair;   // by position; by two positions (the lower one first); 1 outside emit()
+
+    double emit_tables(OpBuffer<T> &ops, const C *due) {
+        const int P = map.n;
+        Ext g;
+        const PassGate *last = nullptr;   // gates of a layer often share their entries
+        Ext z0, z1, c;
+        for (const PassGate *d : gates) {
+            const bool same = last && last->k == d->k && std::equal(d->m, d->m + (1 << d->k), last->m);
+            if (!same) {
+                const Ext i0 = Ext(d->m[0]).inv();
+                z0 = z1 = c = Ext();
+                if (d->m[1] != d->m[0]) z0 = Ext(d->m[1]) * i0;
+                if (d->k == 2) {
+                    if (d->m[2] != d->m[0]) z1 = Ext(d->m[2]) * i0;
+                    if (d->m[3] != d->m[0]) c = Ext(d->m[3]) * i0;
+                    if (!z0.one() || !z1.one()) c = c * (z0 * z1).inv();
+                }
+                last = d;
+            }
+            g = g * Ext(d->m[0]);
+            const int a = d->t[0], b = d->t[1];
+            if (!z0.one()) z[a] = z[a] * z0;
+            if (d->k == 1) continue;
+            if (!z1.one()) z[b] = z[b] * z1;
+            if (!c.one()) {
+                Ext &e = pair[std::min(a, b) * P + std::max(a, b)];
+                e = e.one() ? c : e * c;
+            }
+        }
+        if (due)
+            for (int p = 0; p < P; p++)
+                if (due[p] != C(1.0, 0.0)) {
+                    z[p] = z[p] * Ext(due[p]);
+                    single |= 1ULL << p;
+                }
+        int tile_at[32] = {};
+        uint64_t slots = slot_positions();
+        for (int p = S, k = 0; k < map.n_tile; p++) if (!((slots >> p) & 1)) tile_at[k++] = p;
+        auto of_pair = [&](int p, int q) -> const Ext & { return pair[std::min(p, q) * P + std::max(p, q)]; };
+        double flops = 0;
+        Row row;
+        for (int j = 0; j < map.n_regs; j++) {
+            const int pj = map.slot_pos[j];
+            if (!slot_table(j)) {
+                if (z[pj].one()) continue;
+                PassOp<T> o{};
+                o.kind = PO_DIAG_REG1;
+                o.a = j;
+                o.b = -1;
+                o.c = 1;
+                o.coef[0] = o.coef[1] = {(T)1, (T)0};
+                o.coef[2] = o.coef[3] = {(T)z[pj].re, (T)z[pj].im};
+                o.active = 12u;
+                ops.push_back(o);
+                flops += executed_flops(o);
+                continue;
+            }
+            cx<double> *w = table(ops, j, slot_tile[j], 0, 0, NL + __builtin_popcount(slot_tile[j]));
+            lane_row(z[pj], slot_lane[j], [&](int p) -> const Ext & { return of_pair(p, pj); }, row);
+            put_row(row, w);
+            for (uint32_t m = slot_tile[j]; m; m &= m - 1) put(of_pair(tile_at[__builtin_ctz(m)], pj), w);
+            flops += 3.0;
+        }
+        for (uint64_t m = slot_slot; m; m &= m - 1) {
+            const int j = __builtin_ctzll(m) / 8, k = __builtin_ctzll(m) % 8;
+            const Ext &e = of_pair(map.slot_pos[j], map.slot_pos[k]);
+            PassOp<T> o{};
+            o.kind = PO_DIAG_REG2;
+            o.a = j;
+            o.b = k;
+            o.active = 8u;
+            o.coef[0] = o.coef[1] = o.coef[2] = {(T)1, (T)0};
+            o.coef[3] = {(T)e.re, (T)e.im};
+            ops.push_back(o);
+            flops += executed_flops(o);
+        }
+        if (!has_all()) return flops;
+        uint32_t rows = 0, tt = 0;
+        for (int k = 0; k < map.n_tile; k++) {
+            rows |= (uint32_t)(tile_lane[k] != 0) << k;
+            tt |= (uint32_t)(tile_tile[k] != 0) << k;
+        }
+        const bool tiles = has_tiles();
+        cx<double> *w = table(ops, -1, rows, tiles, tt,
+                              NL * (1 + __builtin_popcount(rows)) + (tiles ? 32 * (1 + __builtin_popcount(tt)) : 0));
+        lane_row(g, (uint32_t)(single & ((1ULL << S) - 1)), [&](int p) -> const Ext & { return z[p]; }, row);
+        for (int p = 0; p < S; p++)
+            for (uint32_t m = lane_lane[p]; m; m &= m - 1) {
+                const int q = __builtin_ctz(m), lo = 1 << p, hi = 1 << q;   // p < q
+                for (int x = hi; x < NL; x += 2 * hi)
+                    for (int y = x + lo; y < x + hi; y += 2 * lo) times(row.re + y, row.im + y, row.re + y, row.im + y, lo, of_pair(p, q));
+            }
+        put_row(row, w);
+        for (uint32_t m = rows; m; m &= m - 1) {
+            const int k = __builtin_ctz(m);
+            lane_row(Ext(), tile_lane[k], [&](int p) -> const Ext & { return of_pair(p, tile_at[k]); }, row);
+            put_row(row, w);
+        }
+        if (tiles) {
+            for (int k = 0; k < 32; k++) put(k < map.n_tile ? z[tile_at[k]] : Ext(), w);
+            for (uint32_t m = tt; m; m &= m - 1) {
+                const int k = __builtin_ctz(m);
+                for (int q = 0; q < 32; q++) put((tile_tile[k] >> q) & 1 ? of_pair(tile_at[k], tile_at[q]) : Ext(), w);
+            }
+        }
+        return flops + 6.0;
+    }
+
+    // (r + i m) f for `cnt` values, f in two parts: one rounding of the
+    // product, none of f's own
+    static void times(const double *r, const double *m, double *ro, double *mo, int cnt, const Ext &f) {
+        const double hr = f.hi().real(), hm = f.hi().imag(), lr = f.lo().real(), lm = f.lo().imag();
+        for (int x = 0; x < cnt; x++) {
+            const double a = r[x], b = m[x];
+            ro[x] = (a * hr - b * hm) + (a * lr - b * lm);
+            mo[x] = (a * hm + b * hr) + (a * lm + b * lr);
+        }
+    }
+    // by lane index x: the scalar times the factors f(p) of its set bits p of mask
+    struct Row {
+        double re[NL], im[NL];
+    };
+    template <typename F> static void lane_row(const Ext &scalar, uint32_t mask, F f, Row &w) {
+        w.re[0] = (double)scalar.re;
+        w.im[0] = (double)scalar.im;
+        for (int p = 0; p < S; p++) {
+            const int half = 1 << p;
+            if ((mask >> p) & 1) {
+                times(w.re, w.im, w.re + half, w.im + half, half, f(p));
+            } else {
+                std::copy(w.re, w.re + half, w.re + half);
+                std::copy(w.im, w.im + half, w.im + half);
+            }
+        }
+    }
+    static void put_row(const Row &r, cx<double> *&w) {
+        for (int x = 0; x < NL; x++) w[x] = {r.re[x], r.im[x]};
+        w += NL;
+    }
+    static void put(const Ext &f, cx<double> *&w) { *w++ = {(double)f.re, (double)f.im}; }
+    // Appends the op and room for its `entries`.
+    static cx<double> *table(OpBuffer<T> &ops, int slot, uint32_t rows, bool tiles, uint32_t tt, int entries) {
+        static_assert(sizeof(PassOp<T>) % sizeof(cx<double>) == 0, "records hold whole table entries");
+        PassOp<T> o{};
+        o.kind = PO_DIAG_TAB;
+        o.a = slot;
+        o.b = tiles;
+        o.c = (int32_t)((entries * sizeof(cx<double>) + sizeof(PassOp<T>) - 1) / sizeof(PassOp<T>));
+        o.active = rows;
+        o.pad[0] = (int32_t)tt;
+        ops.push_back(o);
+        return reinterpret_cast<cx<double> *>(ops.extend(o.c));
+    }
+};
+
 template <typename T, int KH>
 int launch_pass(sq_engine *e, const PassArgs<T> &a) {
     const uint64_t tiles = a.n_tiles * (a.s2 ? 2 : 1);
@@ -377,9 +685,10 @@ int launch_pass(sq_engine *e, const PassArgs<T> &a) {
     return e->check_launch("k_pass");
 }
 
+// tables: runs of diagonal gates may become PO_DIAG_TAB ops
 template <typename T>
 int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredGate> &low,
-                  PlainProgram &prog, void *dst, size_t dst_cap) {
+                  PlainProgram &prog, void *dst, size_t dst_cap, bool tables = true) {
     constexpr int VB = Traits<T>::VB;
     constexpr int S = VB + 6;
     const int n = e->n;
@@ -430,6 +739,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
     const std::vector<sq::SweepStep> &steps = *steps_ptr;
 
     OpBuffer<T> ops(e->ws_ops);
+    DiagRun<T> run(n);
     std::vector<PassGate> lg;
     std::vector<PhaseSplit> sp;
     std::vector<int> fold_into, folded_from, next;
@@ -524,8 +834,10 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
             const PassGate &d = lg[j];
             return any_split && d.cls == OpClass::Diag && d.k == 1 && resident(d.t[0]) && d.m[0] != 0.0;
         };
-        auto flush = [&](int from, bool last) {
-            std::complex<double> fac[64];
+        run.start(regs);
+        // every factor due before gate `from` (see above), by position
+        auto due = [&](int from, std::complex<double> *fac) {
+            std::fill(fac, fac + n, one);
             auto take = [&](int q) {
                 std::complex<double> f = pend[q];
                 pend[q] = one;
@@ -551,7 +863,28 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
             };
             for (int p = 0; p < S; p++) take(p);
             for (int r : regs) take(r);
+        };
+        auto flush = [&](int from, bool last) {
+            std::complex<double> fac[64];
+            due(from, fac);
             l.flops_per_amp += emit_phases<T>(fac, regs, S, last ? gpass : one, ops);
+        };
+        // The diagonal gates that wait, before gate `from`: as tables when that
+        // costs less than one op per gate -- then the phases due go along -- or
+        // one op each.
+        auto settle = [&](int from) {
+            if (run.gates.empty()) return;
+            if (tables && run.gates.size() > 1 && run.cost() < 0.9 * run.old_cost) {
+                std::complex<double> fac[64];
+                if (any_split) due(from, fac);
+                l.flops_per_amp += run.emit(ops, any_split ? fac : nullptr);
+            } else {
+                for (const PassGate *d : run.gates) {
+                    encode_pass_op<T>(*d, regs, ops);
+                    l.flops_per_amp += executed_flops(ops.back());
+                }
+            }
+            run.clear();
         };
         for (size_t i = 0; i < lg.size(); i++) {
             if (fold_into[i] >= 0) continue;   // applied inside the dense gate's op: no work of its own
@@ -571,6 +904,14 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
             if (kSigns && any_split && is_sign_cp(lg[i])) {   // CP(pi): a sign flip
                 ops.push_back(sign_op<T>(lg[i], regs, S));
                 continue;
+            }
+            if (lg[i].cls == OpClass::Diag) {
+                if (unit_diagonal(lg[i])) {
+                    run.add(lg[i]);
+                    continue;
+                }
+            } else if ((run.touched >> lg[i].t[0]) & 1) {
+                settle(i);
             }
             PassGate gi = lg[i];
             if (any_split && gi.cls == OpClass::Dense) {
@@ -622,7 +963,8 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
             }
             l.flops_per_amp += executed_flops(ops.back());
         }
-        if (any_split) flush(lg.size(), true);
+        settle(N);
+        if (any_split) flush(N, true);
         l.n_ops = (int)ops.size() - l.op_begin;
         for (int j = 0; j < kh; j++) l.hpos[j] = regs[j];
         prog.launches.push_back(l);
@@ -641,6 +983,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
         case PO_DIAG_REG1: idx = 5; break;
         case PO_DIAG_REG2: idx = 6; break;
         case PO_PHASES: idx = 7; oi += o.c; break;   // past its coefficient records
+        case PO_DIAG_TAB: idx = o.a < 0 ? 4 : 5; oi += o.c; break;   // past its tables
         case PO_ROT_REG: idx = o.c == 1 ? 3 : 0; break;
         case PO_ROT_LANE: idx = o.a < 4 ? 1 : 2; break;
         case PO_SIGN: idx = o.b == 0 ? 4 : (__builtin_popcount((unsigned)o.b) == 1 ? 5 : 6); break;
@@ -659,6 +1002,9 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
     // upload the program once (in stream order: earlier launches may still read the old one)
     const size_t need = ops.size() * sizeof(PassOp<T>) + 256;
     if (dst) {   // caller-owned buffer: never grown
+        // (tables can take more records than the gates they stand for)
+        if (ops.size() * sizeof(PassOp<T>) > dst_cap && tables)
+            return build_plain_t<T>(e, gates, low, prog, dst, dst_cap, false);
         if (ops.size() * sizeof(PassOp<T>) > dst_cap)
             return e->fail(SQ_ERR_ARG, "the register-pass program (" + std::to_string(ops.size() * sizeof(PassOp<T>)) +
                                            " bytes) exceeds the " + std::to_string(dst_cap) + "-byte scratch");
