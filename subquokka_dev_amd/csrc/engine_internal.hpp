@@ -164,6 +164,12 @@ struct sq_engine {
     // false (g2, l2 untouched) when nothing changes
     bool expand_cnots(const sq_gate *gates, const std::vector<sq::LoweredGate> &low,
                       std::vector<sq_gate> &g2, std::vector<sq::LoweredGate> &l2) const;
+    // A list's SWAPs as a relabelling of the later gates, when register passes
+    // run: sigma[p] = the index bit that then holds bit p.  false (nothing
+    // written) when there are none.
+    bool relabel_swaps(const sq_gate *gates, const std::vector<sq::LoweredGate> &low, std::vector<sq_gate> &g2,
+                       std::vector<sq::LoweredGate> &l2, std::vector<int> &sigma) const;
+    int run_plain(const sq_gate *gates, const std::vector<sq::LoweredGate> &low, void *dst, size_t dst_cap);
     // dst: where the op records go (nullptr: the engine's own growable buffer;
     // otherwise a caller-owned device buffer of dst_cap bytes, never grown)
     int build_plain(const sq_gate *gates, const std::vector<sq::LoweredGate> &low, PlainProgram &prog,
@@ -172,6 +178,7 @@ struct sq_engine {
     // Moves index bit q of the state to bit perm[q] (a permutation of [0, n)
     // keeping the vector bits), out of place through d_alt in one pass.
     int bit_permute(const std::vector<int> &perm);
+    int bit_permute_in_place(const std::vector<int> &perm);
     int setup_scratch();
     int run_plain_program(const PlainProgram &prog, const std::vector<sq::LoweredGate> &low);
     int ensure_partials();

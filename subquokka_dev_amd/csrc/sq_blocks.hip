@@ -127,7 +127,7 @@ int run_blocks_mapped(sq_engine *e, const sq_gate *gates, const std::vector<Lowe
     for (uint64_t b = 0; b < n_blocks; b++) {
         for (size_t i = first; i < first + block_sizes[b]; i++) {
             const sq_gate &g = gates[i];
-            if (g.kind == SQ_GATE_VSWAP_1_1 || g.kind == SQ_GATE_VSWAP_2_2) {
+            if (low[i].cls == OpClass::Perm) {   // VSWAPs, and SWAP gates of the circuit itself
                 // the reference's bit a now holds what its bit b held, and b what a held
                 for (int j = 0; j < low[i].n_pairs; j++) std::swap(sigma[low[i].t[2 * j]], sigma[low[i].t[2 * j + 1]]);
                 continue;
@@ -337,17 +337,28 @@ extern "C" int sq_apply_blocks(sq_engine *e, const sq_gate *gates, const uint32_
                                : run_blocks<float>(e, gates, low, block_sizes, n_blocks);
 }
 
-int sq_engine::bit_permute(const std::vector<int> &perm) {
-    if ((int)perm.size() != n) return fail(SQ_ERR_ARG, "internal: permutation of the wrong size");
+namespace {
+
+// Tile and address tables of a permutation pass.  Source-contiguous low bits
+// [0, c) and the bits that land on the destination's [0, c) make the tile;
+// closed: it also holds every tile bit's image (for an involution) and grows
+// by further bits towards kPermTile.
+// `states`: how many states one launch covers (its grid stays below 2^32
+// threads: wider tiles from 33 bits on).
+int perm_args(sq_engine *e, const std::vector<int> &perm, bool closed, int states, size_t lds_limit, BitPermArgs &a) {
+    const int n = e->n;
+    const int max_groups_bits = 31 - kBlockBits - (states > 1 ? 1 : 0);
+    const int want = std::max(kPermTile, n - max_groups_bits);
+    std::vector<int> inv(n);
     std::vector<char> seen(n, 0);
+    if ((int)perm.size() != n) return e->fail(SQ_ERR_ARG, "internal: permutation of the wrong size");
     for (int q = 0; q < n; q++) {
-        if (perm[q] < 0 || perm[q] >= n || seen[perm[q]]) return fail(SQ_ERR_ARG, "internal: not a permutation");
+        if (perm[q] < 0 || perm[q] >= n || seen[perm[q]]) return e->fail(SQ_ERR_ARG, "internal: not a permutation");
         seen[perm[q]] = 1;
+        inv[perm[q]] = q;
     }
-    int rc = ensure_alt();
-    if (rc) return fail(SQ_ERR_OOM, "no room for the permutation pass's second state buffer");
-    // source-contiguous low bits Ls = [0, c) and the bits that land on the
-    // destination's [0, c); the tile is their union
+    for (int q = 0; closed && q < n; q++)
+        if (inv[q] != perm[q]) return e->fail(SQ_ERR_ARG, "internal: not an involution");
     int c = std::min(6, n);
     std::vector<char> in_t(n, 0);
     auto tile_bits = [&]() {
@@ -357,41 +368,117 @@ int sq_engine::bit_permute(const std::vector<int> &perm) {
             if (q < c || perm[q] < c) { in_t[q] = 1; tb++; }
         return tb;
     };
+    const size_t limit = std::min(lds_limit, e->lds_per_block);
     int tb = tile_bits();
-    while (c > 1 && ((size_t)1 << tb) * amp_bytes() > lds_per_block) { c--; tb = tile_bits(); }
-    if (tb > kPermMaxTile || n - tb > kPermMaxBits || ((size_t)1 << tb) * amp_bytes() > lds_per_block)
-        return fail(SQ_ERR_ARG, "internal: permutation tile too wide");
-    BitPermArgs a{};
+    while (c > 1 && (tb > want || ((size_t)1 << tb) * e->amp_bytes() > limit)) { c--; tb = tile_bits(); }
+    for (int q = 0; q < n; q++) {   // widen a small tile
+        const int more = in_t[q] ? 0 : (closed && perm[q] != q ? 2 : 1);
+        if (!more || tb + more > want || ((size_t)1 << (tb + more)) * e->amp_bytes() > limit) continue;
+        in_t[q] = 1;
+        if (closed) in_t[perm[q]] = 1;
+        tb += more;
+    }
+    if (tb > kPermMaxTile || n - tb > max_groups_bits || ((size_t)1 << tb) * e->amp_bytes() > limit)
+        return e->fail(SQ_ERR_ARG, "internal: permutation tile too wide");
+    a = BitPermArgs{};
     a.tb = tb;
     a.n_other = n - tb;
     std::vector<int> load_pos(n, -1);
     int k = 0;
-    for (int q = 0; q < c; q++) { a.ld_src[k] = q; load_pos[q] = k++; }
-    for (int q = c; q < n; q++) if (in_t[q]) { a.ld_src[k] = q; load_pos[q] = k++; }
-    std::vector<int> inv(n);
-    for (int q = 0; q < n; q++) inv[perm[q]] = q;
+    for (int q = 0; q < n; q++) if (in_t[q]) { a.ld_src[k] = q; load_pos[q] = k++; }
     k = 0;
-    for (int d = 0; d < c; d++) { a.st_loc[k] = load_pos[inv[d]]; a.st_dst[k] = d; k++; }
-    for (int q = 0; q < n; q++)
-        if (in_t[q] && perm[q] >= c) { a.st_loc[k] = load_pos[q]; a.st_dst[k] = perm[q]; k++; }
-    if (k != tb) return fail(SQ_ERR_ARG, "internal: permutation tile bits");
+    for (int d = 0; d < n; d++)   // destination bits ascending
+        if (in_t[inv[d]]) { a.st_loc[k] = load_pos[inv[d]]; a.st_dst[k] = d; k++; }
+    if (k != tb) return e->fail(SQ_ERR_ARG, "internal: permutation tile bits");
     k = 0;
     for (int q = 0; q < n; q++)
         if (!in_t[q]) { a.other_src[k] = q; a.other_dst[k] = perm[q]; k++; }
-    const uint64_t groups = 1ULL << (n - tb);
-    if (groups > 0x7fffffffULL) return fail(SQ_ERR_ARG, "internal: permutation grid");
-    const size_t lds = ((size_t)1 << tb) * amp_bytes();
+    return SQ_OK;
+}
+
+}  // namespace
+
+int sq_engine::bit_permute(const std::vector<int> &perm) {
+    BitPermArgs a;
+    int rc = perm_args(this, perm, false, 1, lds_per_block, a);
+    if (rc) return rc;
+    rc = ensure_alt();
+    if (rc) return fail(SQ_ERR_OOM, "no room for the permutation pass's second state buffer");
+    const unsigned groups = 1u << a.n_other;
+    const size_t lds = ((size_t)1 << a.tb) * amp_bytes();
     const int slot = stat_begin(dtype == SQ_C128 ? "bitperm_c128" : "bitperm_c64", 2.0 * (double)state_bytes());
     if (dtype == SQ_C128)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitperm<double>), (unsigned)groups, kBlock, lds, stream,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitperm<double>), groups, kBlock, lds, stream,
                            static_cast<const cx<double> *>(d_state), static_cast<cx<double> *>(d_alt), a);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitperm<float>), (unsigned)groups, kBlock, lds, stream,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitperm<float>), groups, kBlock, lds, stream,
                            static_cast<const cx<float> *>(d_state), static_cast<cx<float> *>(d_alt), a);
     stat_end(slot);
     rc = check_launch("k_bitperm");
     if (rc) return rc;
     std::swap(d_state, d_alt);   // the state now lives in the other buffer
+    return SQ_OK;
+}
+
+// Moves index bit q of the state (and of d_state2, when set) to bit perm[q],
+// in place: the state keeps its address, which callers may hold.  A cycle is
+// the product of two reflections, so any permutation is at most two
+// involutions, one k_bitswap pass each.  A single transposition is one swap
+// (half a pass); so is each of them when a tile would not fit.
+int sq_engine::bit_permute_in_place(const std::vector<int> &perm) {
+    std::vector<int> part[2] = {std::vector<int>(n), std::vector<int>(n)};
+    for (int q = 0; q < n; q++) part[0][q] = part[1][q] = q;
+    std::vector<char> seen(n, 0);
+    std::vector<std::pair<int, int>> swaps;   // applied in order, they make the permutation
+    for (int q = 0; q < n; q++) {
+        std::vector<int> c;
+        for (int x = q; !seen[x]; x = perm[x]) { seen[x] = 1; c.push_back(x); }
+        const int m = (int)c.size();
+        // c0 -> c1 -> ... : what is at c[m-1] goes to c0 in steps
+        for (int i = m - 1; i > 0; i--) swaps.push_back({std::min(c[0], c[i]), std::max(c[0], c[i])});
+        for (int i = 0; i < m; i++) {
+            part[0][c[i]] = c[(m - i) % m];
+            part[1][c[i]] = c[(m + 1 - i) % m];
+        }
+    }
+    BitPermArgs a[2];
+    bool move[2] = {false, false}, tiles = swaps.size() > 1;
+    for (int k = 0; k < 2; k++) {
+        for (int q = 0; q < n; q++) move[k] = move[k] || part[k][q] != q;
+        if (tiles && move[k]) tiles = perm_args(this, part[k], true, d_state2 ? 2 : 1, lds_per_block / 2, a[k]) == SQ_OK;
+    }
+    if (!tiles) {
+        for (auto &p : swaps) {
+            sq_gate sw{};
+            sw.kind = SQ_GATE_SWAP;
+            sw.nq = 2;
+            sw.q[0] = p.first;
+            sw.q[1] = p.second;
+            LoweredGate lg;
+            int rc = lower(sw, lg);
+            for (int v = 0; !rc && v < (d_state2 ? 2 : 1); v++) {
+                rc = apply_lowered(lg);
+                if (d_state2) std::swap(d_state, d_state2);   // twice: back
+            }
+            if (rc) return rc;
+        }
+        return SQ_OK;
+    }
+    for (int k = 0; k < 2; k++) {
+        if (!move[k]) continue;
+        const unsigned groups = 1u << (a[k].n_other + (d_state2 ? 1 : 0));
+        const size_t lds = ((size_t)2 << a[k].tb) * amp_bytes();
+        const int slot = stat_begin(dtype == SQ_C128 ? "bitswap_c128" : "bitswap_c64",
+                                    2.0 * (double)state_bytes() * (d_state2 ? 2 : 1));
+        if (dtype == SQ_C128)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitswap<double>), groups, kBlock, lds, stream,
+                               static_cast<cx<double> *>(d_state), static_cast<cx<double> *>(d_state2), a[k]);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bitswap<float>), groups, kBlock, lds, stream,
+                               static_cast<cx<float> *>(d_state), static_cast<cx<float> *>(d_state2), a[k]);
+        stat_end(slot);
+        if (int rc = check_launch("k_bitswap")) return rc;
+    }
     return SQ_OK;
 }
 
