@@ -10,6 +10,7 @@
 // accumulated in FP64.
 #pragma once
 #include "common.hpp"
+#include "pass.hpp"
 #include "reduce.hpp"
 
 namespace sqk {
@@ -312,14 +313,160 @@ struct ZTerm {
     uint64_t mask;
 };
 
-// lambda = H psi, and the block partials of <psi|H|psi> (FP64).
-template <typename T>
+// Walsh-Hadamard transform over a wave's 2^KR x 64 values (value index =
+// register * 64 + lane): v[m] <- sum_i (-1)^{popcount(i & m)} v[i], the sums of
+// every sign pattern on 6 + KR bits in 6 + KR additions per value.
+template <int KR> __device__ inline void wave_wht(double (&v)[1 << KR], int lane) {
+    constexpr int R = 1 << KR;
+#pragma unroll
+    for (int b = 0; b < KR; b++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if ((r >> b) & 1) continue;
+            const double x = v[r], y = v[r | (1 << b)];
+            v[r] = x + y;
+            v[r | (1 << b)] = x - y;
+        }
+    const double s0 = (lane & 1) ? -1.0 : 1.0, s1 = (lane & 2) ? -1.0 : 1.0, s2 = (lane & 4) ? -1.0 : 1.0;
+    const double s3 = (lane & 8) ? -1.0 : 1.0, s4 = (lane & 16) ? -1.0 : 1.0, s5 = (lane & 32) ? -1.0 : 1.0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        double x = v[r];
+        x = __builtin_fma(s0, x, lane_xor<1>(x));
+        x = __builtin_fma(s1, x, lane_xor<2>(x));
+        x = __builtin_fma(s2, x, lane_xor<4>(x));
+        x = __builtin_fma(s3, x, lane_xor<8>(x));
+        x = __builtin_fma(s4, x, __shfl_xor(x, 16, 64));
+        x = __builtin_fma(s5, x, __shfl_xor(x, 32, 64));
+        v[r] = x;
+    }
+}
+
+// Gradient terms of a run of diagonal gates.  Their generators are diagonal
+// and the run's gates leave conj(lambda) psi as it is, so every term is a
+// signed sum of the same w_i = Im(conj(lambda_i) psi_i): one read of psi and
+// lambda gives S[mask] = sum_i (-1)^{popcount(i & mask)} w_i for all of the
+// run's masks (a launch per gate reads and writes both: 153 RZZ on 18 qubits
+// in complex128, 153 x 4.5 us -> one launch of 5.4 us).  A wave transforms a
+// tile's w (wave_wht) into LDS; lane l then adds the entries of masks l,
+// l + 64, ... with the sign of the tile's bits.  HBM-bound: the transform is
+// 6 + KR additions per amplitude, whatever the number of masks.
+constexpr int kDiagTermMax = 512;   // masks per launch: eight per lane
+struct DiagTermArgs {
+    uint64_t n_tiles;        // 2^(n - 6 - KR)
+    const uint64_t *tile;    // per mask: its tile-number bits
+    const uint32_t *low;     // per mask: its low 6 + KR bits
+    int n_masks;
+};
+template <typename T, int KR>
+__global__ void __launch_bounds__(kBlock) k_adj_diag_terms(const cx<T> *__restrict__ psi, const cx<T> *__restrict__ lam,
+                                                           const DiagTermArgs a, double *__restrict__ part, uint64_t stride) {
+    constexpr int R = 1 << KR, W = kBlock / 64, NT = R * 64 > kDiagTermMax ? R * 64 : kDiagTermMax;
+    __shared__ double tab[W][NT];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double acc[kDiagTermMax / 64];
+#pragma unroll
+    for (int j = 0; j < kDiagTermMax / 64; j++) acc[j] = 0.0;
+    const uint64_t groups = (a.n_tiles + W - 1) / W;   // every wave of a block makes the same trips
+    for (uint64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+        const uint64_t t = g * W + wv;
+        double v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            v[r] = 0.0;
+            if (t < a.n_tiles) {
+                const uint64_t i = ((t << KR) + r) * 64 + lane;
+                const cx<T> x = psi[i], l = lam[i];
+                v[r] = (double)l.re * (double)x.im - (double)l.im * (double)x.re;
+            }
+        }
+        wave_wht<KR>(v, lane);
+#pragma unroll
+        for (int r = 0; r < R; r++) tab[wv][r * 64 + lane] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kDiagTermMax / 64; j++) {
+            const int k = j * 64 + lane;
+            if (k < a.n_masks) {
+                const double x = tab[wv][a.low[k]];
+                acc[j] += (__popcll(t & a.tile[k]) & 1) ? -x : x;
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < kDiagTermMax / 64; j++) tab[wv][j * 64 + lane] = acc[j];
+    __syncthreads();
+    for (int k = threadIdx.x; k < a.n_masks; k += kBlock) {
+        double x = 0.0;
+        for (int w = 0; w < W; w++) x += tab[w][k];
+        part[k * stride + blockIdx.x] = x;
+    }
+}
+
+// lambda = H psi, and the block partials of <psi|H|psi> (FP64).  On a tile of
+// 2^(6 + KR) amplitudes the tile's bits fix the sign of every string's high
+// part, so the strings that share a low part m add up to one coefficient
+// C[m], and h is the transform of C (wave_wht): the cost per amplitude does not
+// grow with the number of strings (one string per loop trip and amplitude,
+// 39 strings on 26 qubits in complex128: 919 us; so 215 us, one read of the
+// state being 180 us).
+struct ZTermArgs {
+    uint64_t n_tiles;
+    int n_low;               // distinct low parts
+    const uint32_t *low;     // the low part
+    const uint32_t *begin;   // n_low + 1: its strings in the arrays below
+    const double *coef;
+    const uint64_t *tile;    // tile-number bits of a string's mask
+};
+template <typename T, int KR>
 __global__ void __launch_bounds__(kBlock) k_apply_zterms(const cx<T> *__restrict__ psi, cx<T> *__restrict__ lam,
-                                                         const ZTerm *__restrict__ terms, int n_terms, uint64_t n_amp,
-                                                         double *__restrict__ part) {
+                                                         const ZTermArgs a, double *__restrict__ part) {
+    constexpr int R = 1 << KR, W = kBlock / 64;
+    __shared__ double tab[W][R * 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     double acc[1] = {0.0};
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n_amp; i += stride) {
+    const uint64_t groups = (a.n_tiles + W - 1) / W;
+    for (uint64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+        const uint64_t t = g * W + wv;
+        const bool on = t < a.n_tiles;
+        cx<T> x[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            x[r] = {(T)0, (T)0};
+            if (on) x[r] = psi[((t << KR) + r) * 64 + lane];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) tab[wv][r * 64 + lane] = 0.0;
+        __syncthreads();
+        for (int d = lane; d < a.n_low; d += 64) {
+            double c = 0.0;
+            for (uint32_t e = a.begin[d]; e < a.begin[d + 1]; e++)
+                c += (__popcll(t & a.tile[e]) & 1) ? -a.coef[e] : a.coef[e];
+            tab[wv][a.low[d]] = c;
+        }
+        __syncthreads();
+        double h[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) h[r] = tab[wv][r * 64 + lane];
+        __syncthreads();
+        wave_wht<KR>(h, lane);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            acc[0] += h[r] * ((double)x[r].re * (double)x[r].re + (double)x[r].im * (double)x[r].im);
+            if (lam && on) lam[((t << KR) + r) * 64 + lane] = {(T)(h[r] * (double)x[r].re), (T)(h[r] * (double)x[r].im)};
+        }
+    }
+    block_sum<1>(acc, part + blockIdx.x);
+}
+
+// The same for states below one wave (n < 6): every string per amplitude.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_apply_zterms_small(const cx<T> *__restrict__ psi, cx<T> *__restrict__ lam,
+                                                               const ZTerm *__restrict__ terms, int n_terms, uint64_t n_amp,
+                                                               double *__restrict__ part) {
+    double acc[1] = {0.0};
+    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n_amp; i += (uint64_t)gridDim.x * kBlock) {
         double h = 0.0;
         for (int t = 0; t < n_terms; t++) h += (__popcll(i & terms[t].mask) & 1) ? -terms[t].coef : terms[t].coef;
         const cx<T> x = psi[i];
@@ -327,6 +474,20 @@ __global__ void __launch_bounds__(kBlock) k_apply_zterms(const cx<T> *__restrict
         if (lam) lam[i] = {(T)(h * (double)x.re), (T)(h * (double)x.im)};
     }
     block_sum<1>(acc, part + blockIdx.x);
+}
+
+// out[slot] = sum of the slot's `grid` block partials, one wave per slot, in a
+// fixed order (the partials stay on the GPU: 384 parameters x 2048 blocks were
+// 6 MB to copy and add on the host).
+__global__ void __launch_bounds__(kBlock) k_sum_slots(const double *__restrict__ part, uint64_t grid, int n_slots,
+                                                      double *__restrict__ out) {
+    const int slot = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (slot >= n_slots) return;
+    double x = 0.0;
+    for (uint64_t b = lane; b < grid; b += 64) x += part[slot * grid + b];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    if (lane == 0) out[slot] = x;
 }
 
 }  // namespace sqk

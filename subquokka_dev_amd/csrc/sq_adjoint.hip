@@ -15,7 +15,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "subquokka_hip.h"
@@ -243,27 +245,6 @@ int adjoint_gate(const sq_gate &g, sq_gate &out) {
     }
 }
 
-template <typename T>
-int zterms_apply(sq_engine *e, const ZTerm *d_terms, int n_terms, bool to_lambda, double *energy) {
-    const uint64_t na = e->n_amps();
-    const unsigned grid = (unsigned)std::min<uint64_t>(kRedBlocks, std::max<uint64_t>(1, (na + kBlock - 1) / kBlock));
-    int rc = e->ensure_partials();
-    if (rc) return rc;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_apply_zterms<T>), grid, kBlock, 0, e->stream,
-                       reinterpret_cast<const cx<T> *>(e->d_state), to_lambda ? reinterpret_cast<cx<T> *>(e->d_aux) : nullptr,
-                       d_terms, n_terms, na, e->d_part);
-    rc = e->check_launch("k_apply_zterms");
-    if (rc) return rc;
-    std::vector<double> h(grid);
-    hipError_t he = hipMemcpyAsync(h.data(), e->d_part, grid * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-    if (he != hipSuccess) return e->hip_fail(he, "observable partials");
-    double sum = 0;
-    for (double x : h) sum += x;
-    *energy = sum;
-    return SQ_OK;
-}
-
 // Applies a list of gates on the engine's state as register passes (the
 // plain sweep), on psi (lambda_buffer = false) or on lambda.
 int sweep_on(sq_engine *e, const std::vector<sq_gate> &gl, bool on_lambda) {
@@ -286,11 +267,41 @@ int sweep_both(sq_engine *e, const std::vector<sq_gate> &gl) {
     return rc;
 }
 
+// Register bits of a wave tile in the transform kernels: few enough that the
+// tiles fill the GPU (1024 waves at 16 qubits and more), at most 2^4 rows.
+int tile_rows_log2(int n) { return std::max(0, std::min(4, n - 16)); }
+
+template <typename T> struct TransformLaunch {
+    template <int KR> static void terms(sq_engine *e, unsigned grid, const cx<T> *psi, const cx<T> *lam, const DiagTermArgs &a, double *part) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_diag_terms<T, KR>), grid, kBlock, 0, e->stream, psi, lam, a, part, (uint64_t)grid);
+    }
+    template <int KR> static void zterms(sq_engine *e, unsigned grid, const cx<T> *psi, cx<T> *lam, const ZTermArgs &a, double *part) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_apply_zterms<T, KR>), grid, kBlock, 0, e->stream, psi, lam, a, part);
+    }
+};
+
+bool diagonal_kind(int kind) {
+    return kind == SQ_GATE_Z || kind == SQ_GATE_P || kind == SQ_GATE_RZ || kind == SQ_GATE_CP || kind == SQ_GATE_RZZ;
+}
+
+// One step of the reverse sweep.
+struct AdjStep {
+    enum Kind { Inverse, Multi, Gate, Terms, Restore } kind;
+    std::vector<sq_gate> gates;              // Inverse: applied to psi and lambda
+    std::vector<uint64_t> group;             // Multi: its gates, in the sweep's order; Gate: one
+    size_t slot = 0;                         // first partial slot
+    std::vector<uint64_t> masks;             // Terms
+    size_t blob_tile = 0, blob_low = 0;      // Terms: byte offsets of the mask arrays
+    size_t segment = 0;                      // Restore
+};
+
 template <typename T>
 int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, uint64_t ng, const double *theta,
                     uint64_t n_theta, const sq_zterm *terms, uint64_t n_terms, int ckpt_every, double *energy,
                     double *grad) {
     const uint64_t na = e->n_amps();
+    const int n = e->n, kr = tile_rows_log2(n), low_bits = 6 + kr;
+    const bool tiles = n >= 6;   // the transform kernels work on whole waves
     // the circuit with its angles, and the parameterised gates
     std::vector<sq_gate> circ(gates, gates + ng);
     std::vector<uint64_t> pgates;   // indices of parameterised gates, in order
@@ -316,27 +327,227 @@ int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, ui
         for (size_t k = ckpt_every; k < pgates.size(); k += ckpt_every) seg_end.push_back(pgates[k]);
     seg_end.push_back(ng);
     const size_t n_ckpt = grad && ckpt_every > 0 ? seg_end.size() : 0;   // states at the segment starts
+
+    // The reverse sweep's steps.  Parameterised gates give gradient terms as
+    // weighted sums of partial slots (slot 0: the energy):
+    struct Term {
+        int32_t param;
+        size_t slot;
+        double weight;
+    };
+    std::vector<Term> sums;
+    std::vector<AdjStep> steps;
+    size_t n_slots = 1;
+    if (grad) {
+        std::vector<sq_gate> inv_run;       // gates to un-apply before the next term is taken
+        std::vector<uint64_t> group, run;   // pending one-qubit gates of one launch; pending diagonal gates (reverse order)
+        auto flush = [&]() {
+            if (inv_run.empty()) return;
+            AdjStep st{AdjStep::Inverse};
+            st.gates.swap(inv_run);
+            steps.push_back(std::move(st));
+        };
+        auto launch_group = [&]() {
+            if (group.empty()) return;
+            flush();
+            AdjStep st{AdjStep::Multi};
+            st.slot = n_slots;
+            // local bit b: the gate of slot + b, first the earliest in the circuit
+            std::reverse(group.begin(), group.end());
+            for (size_t b = 0; b < group.size(); b++) sums.push_back({param[group[b]], n_slots + b, 1.0});
+            n_slots += group.size();
+            st.group.swap(group);
+            steps.push_back(std::move(st));
+        };
+        auto single = [&](uint64_t gi) {   // two-qubit gate, one launch
+            flush();
+            AdjStep st{AdjStep::Gate};
+            st.slot = n_slots++;
+            st.group = {gi};
+            sums.push_back({param[gi], st.slot, 1.0});
+            steps.push_back(std::move(st));
+        };
+        // Consecutive one-qubit parameterised gates on distinct qubits go to one
+        // k_adj_multi launch: four for complex64 (171 VGPRs), three for complex128
+        const size_t group_max = sizeof(T) == 4 ? 4 : 3;
+        auto add_single_qubit = [&](uint64_t gi) {
+            bool clash = group.size() == group_max;
+            for (uint64_t m : group) clash = clash || circ[m].q[0] == circ[gi].q[0];
+            if (clash) launch_group();
+            group.push_back(gi);
+        };
+        // A run of diagonal gates: all of its terms by one read of psi and lambda,
+        // then its gates join the next un-applies.  Runs that k_adj_multi takes in
+        // one launch (one read and write) stay there.
+        auto close_run = [&]() {
+            if (run.empty()) return;
+            std::vector<uint64_t> r;
+            r.swap(run);
+            size_t n_param = 0;
+            bool one_qubit = true;
+            for (uint64_t gi : r) {
+                n_param += param[gi] >= 0;
+                one_qubit = one_qubit && circ[gi].nq == 1 && param[gi] >= 0;
+            }
+            if (n_param == 0) {
+                launch_group();
+                for (uint64_t gi : r) {
+                    sq_gate inv;
+                    adjoint_gate(circ[gi], inv);
+                    inv_run.push_back(inv);
+                }
+                return;
+            }
+            if (!tiles || (one_qubit && r.size() <= group_max)) {
+                for (uint64_t gi : r) {
+                    if (param[gi] < 0) {
+                        launch_group();
+                        sq_gate inv;
+                        adjoint_gate(circ[gi], inv);
+                        inv_run.push_back(inv);
+                    } else if (circ[gi].nq == 1) {
+                        add_single_qubit(gi);
+                    } else {
+                        launch_group();
+                        single(gi);
+                    }
+                }
+                return;
+            }
+            launch_group();
+            flush();
+            std::vector<uint64_t> masks;
+            std::vector<std::vector<std::pair<int32_t, double>>> weights;   // per mask: (parameter, weight)
+            std::unordered_map<uint64_t, size_t> at;
+            auto use = [&](uint64_t mask, int32_t p, double w) {
+                auto it = at.emplace(mask, masks.size());
+                if (it.second) { masks.push_back(mask); weights.emplace_back(); }
+                weights[it.first->second].push_back({p, w});
+            };
+            for (uint64_t gi : r) {
+                const sq_gate &g = circ[gi];
+                const uint64_t a = 1ULL << g.q[0], b = g.nq > 1 ? 1ULL << g.q[1] : 0;
+                if (param[gi] >= 0) switch (g.kind) {
+                case SQ_GATE_RZ: use(a, param[gi], 1.0); break;
+                case SQ_GATE_RZZ: use(a | b, param[gi], 1.0); break;
+                // -2 Im <lambda|Pi|psi>, Pi = (1 - Z)/2 and (1 - Za)(1 - Zb)/4
+                case SQ_GATE_P: use(0, param[gi], -1.0); use(a, param[gi], 1.0); break;
+                default:
+                    use(0, param[gi], -0.5);
+                    use(a, param[gi], 0.5);
+                    use(b, param[gi], 0.5);
+                    use(a | b, param[gi], -0.5);
+                    break;
+                }
+                sq_gate inv;
+                adjoint_gate(g, inv);
+                inv_run.push_back(inv);
+            }
+            std::vector<sq_gate> after;
+            after.swap(inv_run);   // the launches come first
+            for (size_t m0 = 0; m0 < masks.size(); m0 += kDiagTermMax) {
+                AdjStep st{AdjStep::Terms};
+                const size_t m1 = std::min(masks.size(), m0 + kDiagTermMax);
+                st.masks.assign(masks.begin() + m0, masks.begin() + m1);
+                st.slot = n_slots;
+                for (size_t m = m0; m < m1; m++)
+                    for (auto &w : weights[m]) sums.push_back({w.first, n_slots + (m - m0), w.second});
+                n_slots += m1 - m0;
+                steps.push_back(std::move(st));
+            }
+            inv_run.swap(after);
+        };
+        size_t seg = seg_end.size();   // segments left to sweep back
+        for (uint64_t gi = ng; gi-- > 0;) {
+            // entering the previous segment: psi is re-anchored to the FP64 copy
+            // taken at this segment's end (the next one's start)
+            while (seg > 1 && gi < seg_end[seg - 2]) {
+                close_run();
+                launch_group();
+                flush();
+                AdjStep st{AdjStep::Restore};
+                st.segment = seg - 1;
+                steps.push_back(std::move(st));
+                seg--;
+            }
+            if (diagonal_kind(circ[gi].kind)) {
+                run.push_back(gi);
+                continue;
+            }
+            close_run();
+            if (param[gi] < 0) {
+                launch_group();
+                sq_gate inv;
+                adjoint_gate(circ[gi], inv);
+                inv_run.push_back(inv);
+                continue;
+            }
+            add_single_qubit(gi);
+        }
+        close_run();
+        launch_group();
+        flush();
+    }
+
+    // device buffers: partials, their sums, and the strings' and masks' arrays
     const unsigned grid = (unsigned)std::min<uint64_t>(kRedBlocks, std::max<uint64_t>(1, (na / 2 + kBlock - 1) / kBlock));
-    const size_t term_bytes = n_terms * sizeof(ZTerm);
+    std::vector<unsigned char> blob;
+    auto put = [&](const void *p, size_t bytes) {
+        const size_t at = (blob.size() + 7) / 8 * 8;
+        blob.resize(at + bytes);
+        if (bytes) std::memcpy(blob.data() + at, p, bytes);
+        return at;
+    };
+    const uint64_t low_mask = (1ULL << low_bits) - 1;
+    size_t z_low = 0, z_begin = 0, z_coef = 0, z_tile = 0, z_terms = 0;
+    int n_low = 0;
+    if (tiles) {
+        std::vector<uint32_t> order(n_terms), low, begin;
+        for (uint64_t t = 0; t < n_terms; t++) order[t] = (uint32_t)t;
+        std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+            return (terms[x].mask & low_mask) < (terms[y].mask & low_mask);
+        });
+        std::vector<double> coef;
+        std::vector<uint64_t> tile;
+        for (uint32_t t : order) {
+            const uint32_t l = (uint32_t)(terms[t].mask & low_mask);
+            if (low.empty() || low.back() != l) { low.push_back(l); begin.push_back((uint32_t)coef.size()); }
+            coef.push_back(terms[t].coef);
+            tile.push_back(terms[t].mask >> low_bits);
+        }
+        begin.push_back((uint32_t)coef.size());
+        n_low = (int)low.size();
+        z_low = put(low.data(), low.size() * sizeof(uint32_t));
+        z_begin = put(begin.data(), begin.size() * sizeof(uint32_t));
+        z_coef = put(coef.data(), coef.size() * sizeof(double));
+        z_tile = put(tile.data(), tile.size() * sizeof(uint64_t));
+    } else {
+        std::vector<ZTerm> ht(n_terms);
+        for (uint64_t t = 0; t < n_terms; t++) ht[t] = {terms[t].coef, terms[t].mask};
+        z_terms = put(ht.data(), n_terms * sizeof(ZTerm));
+    }
+    for (auto &st : steps) {
+        if (st.kind != AdjStep::Terms) continue;
+        std::vector<uint64_t> tile;
+        std::vector<uint32_t> low;
+        for (uint64_t m : st.masks) {
+            tile.push_back(m >> low_bits);
+            low.push_back((uint32_t)(m & low_mask));
+        }
+        st.blob_tile = put(tile.data(), tile.size() * sizeof(uint64_t));
+        st.blob_low = put(low.data(), low.size() * sizeof(uint32_t));
+    }
+    const size_t part_bytes = n_slots * grid * sizeof(double), out_bytes = (n_slots * sizeof(double) + 255) / 256 * 256;
     int rc = grad ? ensure(e, &e->d_aux, &e->aux_cap, e->state_bytes(), "hipMalloc(lambda)") : SQ_OK;
     if (!rc && n_ckpt)
         rc = ensure(e, &e->d_ckpt, &e->ckpt_cap, n_ckpt * na * sizeof(cx<double>), "hipMalloc(checkpoints)");
-    if (!rc) rc = ensure(e, &e->d_gradpart, &e->gradpart_cap,
-                         std::max<size_t>(1, pgates.size()) * grid * sizeof(double) + term_bytes + 256,
+    if (!rc) rc = ensure(e, &e->d_gradpart, &e->gradpart_cap, part_bytes + out_bytes + blob.size() + 256,
                          "hipMalloc(gradient partials)");
     if (rc) return rc;
     double *part = static_cast<double *>(e->d_gradpart);
-    ZTerm *d_terms = reinterpret_cast<ZTerm *>(static_cast<char *>(e->d_gradpart) +
-                                               ((std::max<size_t>(1, pgates.size()) * grid * sizeof(double) + 255) / 256) * 256);
-    {
-        std::vector<ZTerm> ht(n_terms);
-        for (uint64_t t = 0; t < n_terms; t++) ht[t] = {terms[t].coef, terms[t].mask};
-        if (n_terms) {
-            hipError_t he = hipMemcpyAsync(d_terms, ht.data(), term_bytes, hipMemcpyHostToDevice, e->stream);
-            if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-            if (he != hipSuccess) return e->hip_fail(he, "observable upload");
-        }
-    }
+    double *d_out = reinterpret_cast<double *>(static_cast<char *>(e->d_gradpart) + part_bytes);
+    char *d_blob = static_cast<char *>(e->d_gradpart) + part_bytes + out_bytes;
+    if ((rc = e->upload(d_blob, blob.data(), blob.size()))) return rc;
     cx<double> *ckpt = n_ckpt ? static_cast<cx<double> *>(e->d_ckpt) : nullptr;
     auto save = [&](size_t slot) {
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_convert<T, double>), e->grid_for(na, kBlock), kBlock, 0, e->stream,
@@ -356,119 +567,107 @@ int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, ui
         if ((rc = sweep_on(e, std::vector<sq_gate>(circ.begin() + begin, circ.begin() + seg_end[sgi]), false))) return rc;
         begin = seg_end[sgi];
     }
-    double en = 0;
-    if ((rc = zterms_apply<T>(e, d_terms, (int)n_terms, grad != nullptr, &en))) return rc;
-    if (energy) *energy = en;
-    if (!grad) return SQ_OK;
+    {
+        const cx<T> *psi = reinterpret_cast<const cx<T> *>(e->d_state);
+        cx<T> *lam = grad ? reinterpret_cast<cx<T> *>(e->d_aux) : nullptr;
+        if (tiles) {
+            const ZTermArgs a{1ULL << (n - low_bits), n_low, reinterpret_cast<const uint32_t *>(d_blob + z_low),
+                              reinterpret_cast<const uint32_t *>(d_blob + z_begin),
+                              reinterpret_cast<const double *>(d_blob + z_coef),
+                              reinterpret_cast<const uint64_t *>(d_blob + z_tile)};
+            switch (kr) {
+            case 0: TransformLaunch<T>::template zterms<0>(e, grid, psi, lam, a, part); break;
+            case 1: TransformLaunch<T>::template zterms<1>(e, grid, psi, lam, a, part); break;
+            case 2: TransformLaunch<T>::template zterms<2>(e, grid, psi, lam, a, part); break;
+            case 3: TransformLaunch<T>::template zterms<3>(e, grid, psi, lam, a, part); break;
+            default: TransformLaunch<T>::template zterms<4>(e, grid, psi, lam, a, part); break;
+            }
+        } else {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_apply_zterms_small<T>), grid, kBlock, 0, e->stream, psi, lam,
+                               reinterpret_cast<const ZTerm *>(d_blob + z_terms), (int)n_terms, na, part);
+        }
+        if ((rc = e->check_launch("k_apply_zterms"))) return rc;
+    }
     // reverse sweep
-    cx<T> *psi = reinterpret_cast<cx<T> *>(e->d_state);
-    cx<T> *lam = reinterpret_cast<cx<T> *>(e->d_aux);
-    size_t seg = seg_end.size();   // segments left to sweep back
-    std::vector<sq_gate> inv_run;
-    auto flush = [&]() {
-        int r = SQ_OK;
-        if (!inv_run.empty()) {
-            r = sweep_both(e, inv_run);
-            inv_run.clear();
-            psi = reinterpret_cast<cx<T> *>(e->d_state);
-            lam = reinterpret_cast<cx<T> *>(e->d_aux);
+    for (const auto &st : steps) {
+        cx<T> *psi = reinterpret_cast<cx<T> *>(e->d_state);
+        cx<T> *lam = reinterpret_cast<cx<T> *>(e->d_aux);
+        double *dst = part + st.slot * grid;
+        switch (st.kind) {
+        case AdjStep::Inverse:
+            if ((rc = sweep_both(e, st.gates))) return rc;
+            break;
+        case AdjStep::Restore:
+            if ((rc = restore(st.segment))) return rc;
+            break;
+        case AdjStep::Multi: {
+            const int M = (int)st.group.size();
+            AdjMultiArgs a{};
+            a.n_items = na >> M;
+            for (int b = 0; b < M; b++) {
+                const sq_gate &g = circ[st.group[b]];
+                a.kind[b] = adj_kind(g.kind);
+                a.q[b] = g.q[0];
+                const double ang = a.kind[b] == ADJ_P ? g.param : g.param / 2;
+                a.c[b] = std::cos(ang);
+                a.s[b] = std::sin(ang);
+            }
+            std::copy(a.q, a.q + M, a.qs);
+            std::sort(a.qs, a.qs + M);
+            const int slot = e->stat_begin("adj_multi", 4.0 * e->amp_bytes() * (double)na);
+            switch (M) {
+            case 1: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 1>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
+            case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 2>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
+            case 3: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 3>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
+            default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 4>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
+            }
+            e->stat_end(slot);
+            if ((rc = e->check_launch("k_adj_multi"))) return rc;
+            break; }
+        case AdjStep::Gate: {
+            const sq_gate &g = circ[st.group[0]];
+            AdjGateArgs a{};
+            a.kind = adj_kind(g.kind);
+            a.n_items = na;
+            a.q0 = g.q[0];
+            a.q1 = g.q[1];
+            const double ang = a.kind == ADJ_CP ? g.param : g.param / 2;
+            a.c = std::cos(ang);
+            a.s = std::sin(ang);
+            // every block writes its partial (zero when it has no items)
+            const int slot = e->stat_begin("adj_gate", 4.0 * e->amp_bytes() * (double)na);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_gate<T>), grid, kBlock, 0, e->stream, psi, lam, a, dst);
+            e->stat_end(slot);
+            if ((rc = e->check_launch("k_adj_gate"))) return rc;
+            break; }
+        case AdjStep::Terms: {
+            const DiagTermArgs a{1ULL << (n - low_bits), reinterpret_cast<const uint64_t *>(d_blob + st.blob_tile),
+                                 reinterpret_cast<const uint32_t *>(d_blob + st.blob_low), (int)st.masks.size()};
+            const int slot = e->stat_begin("adj_diag_terms", 2.0 * e->amp_bytes() * (double)na);
+            switch (kr) {
+            case 0: TransformLaunch<T>::template terms<0>(e, grid, psi, lam, a, dst); break;
+            case 1: TransformLaunch<T>::template terms<1>(e, grid, psi, lam, a, dst); break;
+            case 2: TransformLaunch<T>::template terms<2>(e, grid, psi, lam, a, dst); break;
+            case 3: TransformLaunch<T>::template terms<3>(e, grid, psi, lam, a, dst); break;
+            default: TransformLaunch<T>::template terms<4>(e, grid, psi, lam, a, dst); break;
+            }
+            e->stat_end(slot);
+            if ((rc = e->check_launch("k_adj_diag_terms"))) return rc;
+            break; }
         }
-        return r;
-    };
-    // Consecutive one-qubit parameterised gates on distinct qubits go to one
-    // k_adj_multi launch (up to four in complex64, three in complex128);
-    // two-qubit ones (CP, RZZ) to k_adj_gate.
-    struct Pending {
-        uint64_t gi;
-        size_t pk;   // slot of its gradient partials
-    };
-    std::vector<Pending> group;   // descending pk (the sweep's order)
-    auto launch_group = [&]() -> int {
-        if (group.empty()) return SQ_OK;
-        const int M = (int)group.size();
-        AdjMultiArgs a{};
-        a.n_items = na >> M;
-        for (int b = 0; b < M; b++) {   // local bit b: the b-th smallest partial slot
-            const sq_gate &g = circ[group[M - 1 - b].gi];
-            a.kind[b] = adj_kind(g.kind);
-            a.q[b] = g.q[0];
-            const double ang = a.kind[b] == ADJ_P ? g.param : g.param / 2;
-            a.c[b] = std::cos(ang);
-            a.s[b] = std::sin(ang);
-        }
-        std::copy(a.q, a.q + M, a.qs);
-        std::sort(a.qs, a.qs + M);
-        double *dst = part + group.back().pk * grid;   // slots pk_min .. pk_min + M - 1
-        const int slot = e->stat_begin("adj_multi", 4.0 * e->amp_bytes() * (double)na);
-        switch (M) {
-        case 1: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 1>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
-        case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 2>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
-        case 3: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 3>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
-        default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_multi<T, 4>), grid, kBlock, 0, e->stream, psi, lam, a, dst, (uint64_t)grid); break;
-        }
-        e->stat_end(slot);
-        group.clear();
-        return e->check_launch("k_adj_multi");
-    };
-    size_t pk = pgates.size();
-    for (uint64_t gi = ng; gi-- > 0;) {
-        // entering the previous segment: psi is re-anchored to the FP64 copy
-        // taken at this segment's end (the next one's start)
-        while (seg > 1 && gi < seg_end[seg - 2]) {
-            if ((rc = launch_group())) return rc;
-            if ((rc = flush())) return rc;
-            if ((rc = restore(seg - 1))) return rc;
-            seg--;
-        }
-        if (param[gi] < 0) {
-            if ((rc = launch_group())) return rc;
-            sq_gate inv;
-            adjoint_gate(circ[gi], inv);
-            inv_run.push_back(inv);
-            continue;
-        }
-        if ((rc = flush())) return rc;
-        pk--;
-        const sq_gate &g = circ[gi];
-        const int kind = adj_kind(g.kind);
-        if (kind != ADJ_CP && kind != ADJ_RZZ) {
-            // four gates per launch for complex64 (171 VGPRs), three for complex128
-            bool clash = group.size() == (sizeof(T) == 4 ? 4u : 3u);
-            for (const auto &m : group) clash = clash || circ[m.gi].q[0] == g.q[0];
-            if (clash && (rc = launch_group())) return rc;
-            group.push_back({gi, pk});
-            continue;
-        }
-        if ((rc = launch_group())) return rc;
-        AdjGateArgs a{};
-        a.kind = kind;
-        a.n_items = na;
-        a.q0 = g.q[0];
-        a.q1 = g.q[1];
-        const double ang = a.kind == ADJ_CP ? g.param : g.param / 2;
-        a.c = std::cos(ang);
-        a.s = std::sin(ang);
-        // every block writes its partial (zero when it has no items)
-        const int slot = e->stat_begin("adj_gate", 4.0 * e->amp_bytes() * (double)na);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_adj_gate<T>), grid, kBlock, 0, e->stream, psi, lam, a, part + pk * grid);
-        e->stat_end(slot);
-        if ((rc = e->check_launch("k_adj_gate"))) return rc;
     }
-    if ((rc = launch_group())) return rc;
-    if ((rc = flush())) return rc;
     if (ckpt && (rc = restore(0))) return rc;   // the state the call started from, exactly
-    std::vector<double> h(pgates.size() * grid);
-    if (!h.empty()) {
-        hipError_t he = hipMemcpyAsync(h.data(), part, h.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-        if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-        if (he != hipSuccess) return e->hip_fail(he, "gradient partials");
-    }
+    hipLaunchKernelGGL(k_sum_slots, (unsigned)((n_slots + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, e->stream,
+                       (const double *)part, (uint64_t)grid, (int)n_slots, d_out);
+    if ((rc = e->check_launch("k_sum_slots"))) return rc;
+    std::vector<double> h(n_slots);
+    hipError_t he = hipMemcpyAsync(h.data(), d_out, n_slots * sizeof(double), hipMemcpyDeviceToHost, e->stream);
+    if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
+    if (he != hipSuccess) return e->hip_fail(he, "gradient sums");
+    if (energy) *energy = h[0];
+    if (!grad) return SQ_OK;
     std::fill(grad, grad + n_theta, 0.0);
-    for (size_t k = 0; k < pgates.size(); k++) {
-        double sum = 0;
-        for (unsigned b = 0; b < grid; b++) sum += h[k * grid + b];
-        grad[param[pgates[k]]] += sum;
-    }
+    for (const Term &t : sums) grad[t.param] += t.weight * h[t.slot];
     return SQ_OK;
 }
 

@@ -560,6 +560,7 @@ private:
         auto of_pair = [&](int p, int q) -> const Ext & { return pair[std::min(p, q) * P + std::max(p, q)]; };
         double flops = 0;
         Row row;
+        Ext carry;
         for (int j = 0; j < map.n_regs; j++) {
             const int pj = map.slot_pos[j];
             if (!slot_table(j)) {
@@ -579,7 +580,7 @@ private:
             cx<double> *w = table(ops, j, slot_tile[j], 0, 0, NL + __builtin_popcount(slot_tile[j]));
             lane_row(z[pj], slot_lane[j], [&](int p) -> const Ext & { return of_pair(p, pj); }, row);
             put_row(row, w);
-            for (uint32_t m = slot_tile[j]; m; m &= m - 1) put(of_pair(tile_at[__builtin_ctz(m)], pj), w);
+            for (uint32_t m = slot_tile[j]; m; m &= m - 1) put_carry(of_pair(tile_at[__builtin_ctz(m)], pj), w, carry);
             flops += 3.0;
         }
         for (uint64_t m = slot_slot; m; m &= m - 1) {
@@ -621,7 +622,10 @@ private:
             for (int k = 0; k < 32; k++) put(k < map.n_tile ? z[tile_at[k]] : Ext(), w);
             for (uint32_t m = tt; m; m &= m - 1) {
                 const int k = __builtin_ctz(m);
-                for (int q = 0; q < 32; q++) put((tile_tile[k] >> q) & 1 ? of_pair(tile_at[k], tile_at[q]) : Ext(), w);
+                for (int q = 0; q < 32; q++) {
+                    if ((tile_tile[k] >> q) & 1) put_carry(of_pair(tile_at[k], tile_at[q]), w, carry);
+                    else put(Ext(), w);
+                }
             }
         }
         return flops + 6.0;
@@ -659,6 +663,15 @@ private:
         w += NL;
     }
     static void put(const Ext &f, cx<double> *&w) { *w++ = {(double)f.re, (double)f.im}; }
+    // The same for factors that are often equal and whose product over a subset
+    // is taken: each entry takes along what the entries before it lost to
+    // rounding, so equal factors do not all err the same way.
+    static void put_carry(const Ext &f, cx<double> *&w, Ext &carry) {
+        const Ext v = f * carry;
+        const std::complex<double> r = v.hi();
+        carry = v * Ext(r).inv();
+        *w++ = {r.real(), r.imag()};
+    }
     // Appends the op and room for its `entries`.
     static cx<double> *table(OpBuffer<T> &ops, int slot, uint32_t rows, bool tiles, uint32_t tt, int entries) {
         static_assert(sizeof(PassOp<T>) % sizeof(cx<double>) == 0, "records hold whole table entries");

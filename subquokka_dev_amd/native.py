@@ -180,17 +180,18 @@ def parse_circuit(text, n, is_subcircuit=False):
     L = lib()
     ng, nb, el = ctypes.c_uint64(0), ctypes.c_uint64(0), ctypes.c_int32(0)
     raw = text.encode() if isinstance(text, str) else text
-    rc = L.sq_parse_circuit(raw, n, int(is_subcircuit), None, 0, ctypes.byref(ng), None, 0, ctypes.byref(nb),
-                            ctypes.byref(el))
-    if rc not in (SQ_OK, SQ_ERR_ARG):
-        raise SqError(rc, f"parse error at line {el.value}")
-    gates = (SqGate * max(1, ng.value))()
-    blocks = (ctypes.c_uint32 * max(1, nb.value))()
-    rc = L.sq_parse_circuit(raw, n, int(is_subcircuit), gates, ng.value, ctypes.byref(ng),
-                            blocks if is_subcircuit else None, nb.value if is_subcircuit else 0,
+    cap = raw.count(b"\n") + 1   # at most one gate or block a line: the text is read once
+    gates = (SqGate * cap)()
+    blocks = (ctypes.c_uint32 * cap)()
+    rc = L.sq_parse_circuit(raw, n, int(is_subcircuit), gates, cap, ctypes.byref(ng),
+                            blocks if is_subcircuit else None, cap if is_subcircuit else 0,
                             ctypes.byref(nb), ctypes.byref(el))
     if rc != SQ_OK:
         raise SqError(rc, f"parse error at line {el.value}")
+    if ng.value != cap:
+        gates = (SqGate * max(1, ng.value)).from_buffer(gates)   # the same memory, as long as the list
+    if nb.value != cap:
+        blocks = (ctypes.c_uint32 * max(1, nb.value)).from_buffer(blocks)
     return gates, (blocks if is_subcircuit else None), ng.value, nb.value
 
 
