@@ -91,6 +91,7 @@ struct sq_engine {
     void *d_scratch = nullptr;      // this device's static scratch array (sq_apply_gates_noalloc)
     int sweep_mode = 0;             // 0: register passes, 1: one launch per gate
     int pass_qbits = 5;             // register qubits per pass (1..5; set by sq_create)
+    bool keep_order = false;        // register passes round every gate where the list has it (set per call)
     int lane_moves = 3;             // top lane positions a pass may give to other qubits (0..3)
     int plan_beam = sq::kDefaultPlanBeam;   // register-pass planner: sets kept per size (1: greedy)
     bool phase_split = true;        // register passes: one-qubit dense gates as phase, real rotation, phase
@@ -160,8 +161,8 @@ struct sq_engine {
     int apply_plain(const sq_gate *gates, size_t n_gates, const std::vector<sq::LoweredGate> &low);
     // lowers a list into ws_low; the message names the gate that fails
     int lower_list(const sq_gate *gates, size_t n_gates);
-    // CNOTs (exact U2 permutation matrices) as H CZ H when register passes run;
-    // false (g2, l2 untouched) when nothing changes
+    // CNOTs (exact U2 permutation matrices) as H CZ H (keep_order); false
+    // (g2, l2 untouched) when nothing changes
     bool expand_cnots(const sq_gate *gates, const std::vector<sq::LoweredGate> &low,
                       std::vector<sq_gate> &g2, std::vector<sq::LoweredGate> &l2) const;
     // A list's SWAPs as a relabelling of the later gates, when register passes

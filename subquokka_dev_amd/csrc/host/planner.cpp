@@ -135,32 +135,37 @@ std::vector<PlanPass> plan_passes(const std::vector<sq_gate> &gates, int n, int 
 
 namespace {
 
-// Gates of `pending` that a register pass with resident qubit set `in` can
-// run, in order.  Stops once every qubit is blocked.
-int count_pass(const std::vector<sq_gate> &gates, const std::vector<int> &pending, const std::vector<char> &in,
-               const std::vector<char> &mergeable, const std::vector<char> &anywhere, std::vector<char> &blocked,
-               std::vector<int> *out, int *dense = nullptr) {
-    std::fill(blocked.begin(), blocked.end(), 0);
-    const int n = (int)blocked.size();
-    int cnt = 0, n_blocked = 0, n_dense = 0;
-    for (int gi : pending) {
-        const sq_gate &g = gates[gi];
-        bool ok = mergeable[gi] != 0;
-        for (int i = 0; ok && i < g.nq; i++)
-            if (blocked[g.q[i]] || (!anywhere[gi] && !in[g.q[i]])) ok = false;
-        if (ok) {
-            cnt++;
-            n_dense += !anywhere[gi];
-            if (out) out->push_back(gi);
-            continue;
-        }
-        for (int i = 0; i < g.nq; i++)
-            if (!blocked[g.q[i]]) { blocked[g.q[i]] = 1; n_blocked++; }
-        if (n_blocked == n) break;
+// count_pass on qubit bit masks (n <= 64), for the planner's inner loop: the
+// gates of `pending` a pass with resident set `in` can run, stopping once
+// every qubit is blocked.
+struct MaskCounter {
+    std::vector<uint64_t> qmask;   // per gate: its qubits
+    const std::vector<char> &mergeable;
+    const std::vector<uint64_t> &need;
+    uint64_t all;
+    MaskCounter(const std::vector<sq_gate> &gates, const std::vector<char> &m, const std::vector<uint64_t> &nd, int n)
+        : qmask(gates.size()), mergeable(m), need(nd), all(n >= 64 ? ~0ULL : (1ULL << n) - 1) {
+        for (size_t i = 0; i < gates.size(); i++)
+            for (int j = 0; j < gates[i].nq; j++) qmask[i] |= 1ULL << gates[i].q[j];
     }
-    if (dense) *dense = n_dense;
-    return cnt;
-}
+    int count(const std::vector<int> &pending, uint64_t in, int *dense, std::vector<int> *out = nullptr) const {
+        uint64_t blocked = 0;
+        int cnt = 0, n_dense = 0;
+        for (int gi : pending) {
+            const uint64_t m = qmask[gi];
+            if (mergeable[gi] && !(m & blocked) && !(need[gi] & ~in)) {
+                cnt++;
+                n_dense += need[gi] != 0;
+                if (out) out->push_back(gi);
+                continue;
+            }
+            blocked |= m;
+            if (blocked == all) break;
+        }
+        *dense = n_dense;
+        return cnt;
+    }
+};
 
 }  // namespace
 
@@ -275,51 +280,16 @@ int lane_cost(const std::vector<int> &lanes, const std::vector<int> &dense_cnt, 
 
 }  // namespace
 
-namespace {
-
-// count_pass on qubit bit masks (n <= 64), for the planner's inner loop: the
-// gates of `pending` a pass with resident set `in` can run, stopping once
-// every qubit is blocked.
-struct MaskCounter {
-    std::vector<uint64_t> qmask;   // per gate: its qubits
-    const std::vector<char> &mergeable, &anywhere;
-    uint64_t all;
-    MaskCounter(const std::vector<sq_gate> &gates, const std::vector<char> &m, const std::vector<char> &a, int n)
-        : qmask(gates.size()), mergeable(m), anywhere(a), all(n >= 64 ? ~0ULL : (1ULL << n) - 1) {
-        for (size_t i = 0; i < gates.size(); i++)
-            for (int j = 0; j < gates[i].nq; j++) qmask[i] |= 1ULL << gates[i].q[j];
-    }
-    int count(const std::vector<int> &pending, uint64_t in, int *dense) const {
-        uint64_t blocked = 0;
-        int cnt = 0, n_dense = 0;
-        for (int gi : pending) {
-            const uint64_t m = qmask[gi];
-            if (mergeable[gi] && !(m & blocked) && (anywhere[gi] || !(m & ~in))) {
-                cnt++;
-                n_dense += !anywhere[gi];
-                continue;
-            }
-            blocked |= m;
-            if (blocked == all) break;
-        }
-        *dense = n_dense;
-        return cnt;
-    }
-};
-
-}  // namespace
-
 std::vector<SweepStep> plan_register_passes(const std::vector<sq_gate> &gates, const std::vector<char> &mergeable,
-                                            const std::vector<char> &anywhere, int n, int low, int kh, int nlh,
+                                            const std::vector<uint64_t> &need, int n, int low, int kh, int nlh,
                                             int lh_max, int beam) {
     std::vector<SweepStep> steps;
     std::vector<int> pending(gates.size());
     for (size_t i = 0; i < gates.size(); i++) pending[i] = (int)i;
-    std::vector<char> in(n), blocked(n);
     if (nlh < 0 || nlh > low) nlh = 0;
     const int fixed = std::min(low - nlh, n);
     const int lo = low - nlh;
-    const MaskCounter counter(gates, mergeable, anywhere, n);
+    const MaskCounter counter(gates, mergeable, need, n);
     const uint64_t lane_pos = nlh ? (((1ULL << nlh) - 1) << lo) : 0;
     const uint64_t lane_ok = lh_max >= 63 ? ~0ULL : (lh_max < 0 ? 0 : (2ULL << lh_max) - 1);
     // Whether a chosen set fits kh register slots plus the free lane positions
@@ -342,13 +312,8 @@ std::vector<SweepStep> plan_register_passes(const std::vector<sq_gate> &gates, c
             pending.erase(pending.begin());
             continue;
         }
-        std::fill(in.begin(), in.end(), 0);
-        for (int q = 0; q < fixed; q++) in[q] = 1;
-        if (nlh == 0) {
-            for (int q = fixed; q < std::min(low, n); q++) in[q] = 1;
-        }
         uint64_t in_mask = 0;
-        for (int q = 0; q < n; q++) if (in[q]) in_mask |= 1ULL << q;
+        for (int q = 0; q < (nlh == 0 ? std::min(low, n) : fixed); q++) in_mask |= 1ULL << q;
         // dense gates per qubit among the pending ones, for the lane choice
         std::vector<int> dense_cnt(n, 0);
         // Beam search over the chosen qubits: keep the `beam` best sets at each
@@ -395,29 +360,29 @@ std::vector<SweepStep> plan_register_passes(const std::vector<sq_gate> &gates, c
         // gates run on any qubit)
         std::vector<int> chosen;
         {
-            for (int x : states[0].chosen) in[x] = 1;
             std::vector<int> sel;
-            count_pass(gates, pending, in, mergeable, anywhere, blocked, &sel);
-            std::vector<char> used(n, 0);
-            for (int gi : sel)
-                if (!anywhere[gi])
-                    for (int i = 0; i < gates[gi].nq; i++) used[gates[gi].q[i]] = 1;
-            for (int x : states[0].chosen) {
-                if (used[x]) chosen.push_back(x);
-                else in[x] = 0;
-            }
+            int dense = 0;
+            counter.count(pending, in_mask | states[0].mask, &dense, &sel);
+            uint64_t used = 0;
+            for (int gi : sel) used |= need[gi];
+            for (int x : states[0].chosen)
+                if ((used >> x) & 1) chosen.push_back(x);
         }
         SweepStep st;
         st.merged = true;
-        count_pass(gates, pending, in, mergeable, anywhere, blocked, &st.gates);
+        {
+            uint64_t in = in_mask;
+            int dense = 0;
+            for (int x : chosen) in |= 1ULL << x;
+            counter.count(pending, in, &dense, &st.gates);
+        }
         if (st.gates.empty()) {   // cannot happen for a mergeable first gate; stay safe
             st.merged = false;
             st.gates.push_back(g0);
         }
         if (nlh) {
             for (int gi : st.gates)
-                if (!anywhere[gi])
-                    for (int i = 0; i < gates[gi].nq; i++) dense_cnt[gates[gi].q[i]]++;
+                for (uint64_t m = need[gi]; m; m &= m - 1) dense_cnt[__builtin_ctzll(m)]++;
             if (!assign_lanes(chosen, dense_cnt, lo, nlh, kh, lh_max, &st.regs, &st.lanes)) {
                 // unreachable: every chosen set was checked; fall back to one gate
                 st = SweepStep{};
@@ -554,14 +519,19 @@ extern "C" int sq_plan(const char *circuit_text, int32_t n, int32_t mode, int32_
         // param + 3 chosen qubits (param in registers, up to three in the top
         // lane positions); other gates stand alone
         if (param < 1 || param > 5) return SQ_ERR_ARG;
-        std::vector<char> mergeable(gates.size(), 0), anywhere(gates.size(), 0);
+        std::vector<char> mergeable(gates.size(), 0);
+        std::vector<uint64_t> need(gates.size(), 0);
         for (size_t i = 0; i < gates.size(); i++) {
             sq::LoweredGate lg;
             if (sq::lower_gate(gates[i], n, lg, nullptr) != SQ_OK) return SQ_ERR_ARG;
-            if (lg.cls == sq::OpClass::Diag && lg.k <= 2) mergeable[i] = anywhere[i] = 1;
-            else if (lg.cls == sq::OpClass::Dense && lg.k == 1) mergeable[i] = 1;
+            if (lg.cls == sq::OpClass::Diag && lg.k <= 2) {
+                mergeable[i] = 1;
+            } else if (lg.cls == sq::OpClass::Dense && lg.k == 1) {
+                mergeable[i] = 1;
+                need[i] = 1ULL << lg.t[0];
+            }
         }
-        for (auto &st : sq::plan_register_passes(gates, mergeable, anywhere, n, 6, param, 3, std::min(n - 1, 27),
+        for (auto &st : sq::plan_register_passes(gates, mergeable, need, n, 6, param, 3, std::min(n - 1, 27),
                                                  sq::kDefaultPlanBeam)) {
             out += std::to_string(st.gates.size()) + "\n";
             for (int gi : st.gates) out += sq::gate_to_line(gates[gi]) + "\n";

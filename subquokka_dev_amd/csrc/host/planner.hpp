@@ -34,8 +34,9 @@ std::vector<PlanPass> plan_passes(const std::vector<sq_gate> &gates, int n, int 
 // other qubits instead (at most lh_max): the step then has [0, low - nlh)
 // plus up to kh + nlh chosen qubits resident.
 //   mergeable[i]: gate i may run inside a register pass;
-//   anywhere[i]:  gate i may run whatever the pass's qubit set (diagonal
-//                 gates: the phase needs only the amplitude's index).
+//   need[i]:      the qubits gate i needs resident (all of a dense gate's, a
+//                 CNOT's target; none of a diagonal gate's: the phase needs
+//                 only the amplitude's index).
 // Per-qubit order is kept: a gate joins a step only after every earlier
 // gate sharing a qubit with it.
 struct SweepStep {
@@ -49,7 +50,7 @@ struct SweepStep {
 // passes from 25 (greedy) to 19.
 constexpr int kDefaultPlanBeam = 16;
 std::vector<SweepStep> plan_register_passes(const std::vector<sq_gate> &gates, const std::vector<char> &mergeable,
-                                            const std::vector<char> &anywhere, int n, int low, int kh,
+                                            const std::vector<uint64_t> &need, int n, int low, int kh,
                                             int nlh = 0, int lh_max = -1, int beam = 1);
 
 // Reference subcircuit text (finder.cpp:69-333 format) for a chunk of

@@ -11,6 +11,8 @@
 //
 // Gates a pass can hold:
 //   * dense one-qubit gates on a vector, lane or register bit (H X Y U1 RX RY);
+//   * CNOTs whose target is a vector, lane or register bit, the control on
+//     ANY qubit (an exact exchange of amplitudes);
 //   * diagonal one- and two-qubit gates on ANY qubits (Z P RZ CP RZZ): the
 //     phase depends only on the amplitude's global index, which every lane
 //     knows.
@@ -68,6 +70,10 @@ enum PassOpKind : int32_t {
     PO_SIGN = 11,        // amplitude i negated where every bit of i named below is 1 (CP(pi),
                          //   CZ): a = mask of virtual positions < VB + 6, b = mask of register
                          //   slots, pad[0], pad[1] = tile positions (-1: none)
+    PO_CNOT = 13,        // amplitudes exchanged along a position where a control bit is 1.  Target:
+                         //   b = 0 register slot a, 1 lane bit a, 2 the complex64 vector.
+                         //   Control: active = 0 register slot c, 1 position c below VB + 6,
+                         //   2 tile position c
     PO_DIAG_TAB = 12,    // a run of diagonal gates in one product: amplitude i times F(i) when
                          //   bit a of its register index is 1 (a < 0: every amplitude), F from
                          //   complex<double> tables in the c records after the op:
@@ -683,6 +689,48 @@ __device__ inline void pass_diag_reg2(Pack<T> (&v)[R], const Coef4<T> d, uint32_
     }
 }
 
+// The value of lane ^ MASK.
+template <int MASK, typename T> __device__ inline T lane_partner(T x, int lane) {
+    if constexpr (MASK <= 8) {
+        return lane_xor<MASK>(x);
+    } else {   // both halves of a swap of x with itself: the lower (upper) rows twice
+        T a = x, b = x;
+        permlane_swap<MASK>(a, b);
+        return (lane & MASK) ? a : b;
+    }
+}
+
+// PO_CNOT.  on[e]: the lane's control (per vector element); cslot >= 0: the
+// control is that register bit instead.  Moves and selects only.
+template <typename T, int J, int R, int E>
+__device__ inline void pass_cnot_reg(Pack<T> (&v)[R], const bool (&on)[E], int cslot) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if ((r >> J) & 1) continue;
+        if (cslot >= 0 && !((r >> cslot) & 1)) continue;   // wave-uniform
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            cx<T> &x = v[r].e[e], &y = v[r | (1 << J)].e[e];
+            const cx<T> p = x;
+            x = csel(on[e], y, x);
+            y = csel(on[e], p, y);
+        }
+    }
+}
+template <typename T, int MASK, int R, int E>
+__device__ inline void pass_cnot_lane(Pack<T> (&v)[R], const bool (&on)[E], int cslot, int lane) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (cslot >= 0 && !((r >> cslot) & 1)) continue;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            cx<T> &x = v[r].e[e];
+            const cx<T> p = {lane_partner<MASK>(x.re, lane), lane_partner<MASK>(x.im, lane)};
+            x = csel(on[e], p, x);
+        }
+    }
+}
+
 // PO_DIAG_TAB's factor of one lane and vector element.  One gate costs a pass
 // four FP64 products per register it touches; here the gates that share a
 // register slot (or none) first meet in one factor per lane -- a table entry
@@ -905,6 +953,39 @@ __global__ void __launch_bounds__(kBlock) k_pass(cx<T> *__restrict__ s, const Pa
                     if ((r & o.b) == o.b)
 #pragma unroll
                         for (int e = 0; e < E; e++) flip_sign(v[r].e[e], mk[e]);
+                break; }
+            case PO_CNOT: {
+                if (o.active == 2 && !((tb >> o.c) & 1)) break;   // the wave's control is 0
+                const int cslot = o.active == 0 ? o.c : -1;
+                bool on[E];
+#pragma unroll
+                for (int e = 0; e < E; e++) on[e] = o.active != 1 || (((base + e) >> o.c) & 1);
+                if (o.b == 2) {
+                    if constexpr (E == 2) {
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            if (cslot >= 0 && !((r >> cslot) & 1)) continue;
+                            const cx<T> p = v[r].e[0];
+                            v[r].e[0] = csel(on[0], v[r].e[1], p);
+                            v[r].e[1] = csel(on[0], p, v[r].e[1]);
+                        }
+                    }
+                    break;
+                }
+                switch (o.b * 8 + o.a) {
+                case 0: pass_cnot_reg<T, 0, R, E>(v, on, cslot); break;
+                case 1: if constexpr (KH > 1) pass_cnot_reg<T, 1, R, E>(v, on, cslot); break;
+                case 2: if constexpr (KH > 2) pass_cnot_reg<T, 2, R, E>(v, on, cslot); break;
+                case 3: if constexpr (KH > 3) pass_cnot_reg<T, 3, R, E>(v, on, cslot); break;
+                case 4: if constexpr (KH > 4) pass_cnot_reg<T, 4, R, E>(v, on, cslot); break;
+                case 8: pass_cnot_lane<T, 1, R, E>(v, on, cslot, lane); break;
+                case 9: pass_cnot_lane<T, 2, R, E>(v, on, cslot, lane); break;
+                case 10: pass_cnot_lane<T, 4, R, E>(v, on, cslot, lane); break;
+                case 11: pass_cnot_lane<T, 8, R, E>(v, on, cslot, lane); break;
+                case 12: pass_cnot_lane<T, 16, R, E>(v, on, cslot, lane); break;
+                case 13: pass_cnot_lane<T, 32, R, E>(v, on, cslot, lane); break;
+                default: break;
+                }
                 break; }
             case PO_DIAG_TAB: {
                 const DiagTab<E> tab{reinterpret_cast<const cx<double> *>(a.ops + op + 1), lane};

@@ -302,6 +302,15 @@ int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, ui
     const uint64_t na = e->n_amps();
     const int n = e->n, kr = tile_rows_log2(n), low_bits = 6 + kr;
     const bool tiles = n >= 6;   // the transform kernels work on whole waves
+    // complex64: each gate is un-applied and its term taken where the list has
+    // it, so that the FP32 rounding, and with it the gradient to all digits,
+    // stays what it is (see keep_order)
+    const bool runs = tiles && sizeof(T) == 8;
+    struct KeepOrder {
+        sq_engine *e;
+        KeepOrder(sq_engine *x, bool on) : e(x) { e->keep_order = on; }
+        ~KeepOrder() { e->keep_order = false; }
+    } keep(e, sizeof(T) == 4);
     // the circuit with its angles, and the parameterised gates
     std::vector<sq_gate> circ(gates, gates + ng);
     std::vector<uint64_t> pgates;   // indices of parameterised gates, in order
@@ -398,7 +407,7 @@ int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, ui
                 }
                 return;
             }
-            if (!tiles || (one_qubit && r.size() <= group_max)) {
+            if (!runs || (one_qubit && r.size() <= group_max)) {
                 for (uint64_t gi : r) {
                     if (param[gi] < 0) {
                         launch_group();

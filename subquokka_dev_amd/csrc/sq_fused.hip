@@ -238,9 +238,11 @@ int plan_fused_passes(sq_engine *e, const std::vector<sq_gate> &gates, const std
                       FusedPassPlan &plan) {
     const int n = e->n;
     const size_t ng = gates.size();
-    std::vector<char> mergeable(ng, 1), anywhere(ng, 0);
-    for (size_t i = 0; i < ng; i++) anywhere[i] = low[i].cls == OpClass::Diag;
-    const auto steps = sq::plan_register_passes(gates, mergeable, anywhere, n, 4, r - 4, 0, -1, e->plan_beam);
+    std::vector<char> mergeable(ng, 1);
+    std::vector<uint64_t> need(ng, 0);
+    for (size_t i = 0; i < ng; i++)
+        for (int j = 0; low[i].cls != OpClass::Diag && j < gates[i].nq; j++) need[i] |= 1ULL << gates[i].q[j];
+    const auto steps = sq::plan_register_passes(gates, mergeable, need, n, 4, r - 4, 0, -1, e->plan_beam);
     plan = FusedPassPlan{};
     plan.r = r;
     for (const auto &st : steps) {

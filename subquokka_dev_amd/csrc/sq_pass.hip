@@ -69,11 +69,30 @@ private:
     }
 };
 
-// A gate of a register pass: dense on one qubit or diagonal on one or two, in
-// the pass's virtual positions (t ascending).
+// The target of a U2 whose matrix is exactly a CNOT (control either qubit; the
+// reference's way to write one), or -1.  Local index bit 0 is t[0], bit 1 is t[1].
+int cnot_target(const LoweredGate &g) {
+    if (g.cls != OpClass::Dense || g.k != 2) return -1;
+    const std::complex<double> one(1.0, 0.0), zero(0.0, 0.0);
+    auto is = [&](const int *perm) {   // row r has its one at column perm[r]
+        for (int r = 0; r < 4; r++)
+            for (int c = 0; c < 4; c++)
+                if (g.m[r * 4 + c] != (c == perm[r] ? one : zero)) return false;
+        return true;
+    };
+    static const int flip1[4] = {0, 3, 2, 1};   // control t[0]: bit 1 flips where bit 0 is set
+    static const int flip0[4] = {0, 1, 3, 2};   // control t[1]: bit 0 flips where bit 1 is set
+    if (is(flip1)) return g.t[1];
+    if (is(flip0)) return g.t[0];
+    return -1;
+}
+
+// A gate of a register pass: dense on one qubit, diagonal on one or two (t
+// ascending) or a CNOT (t: target, control), in the pass's virtual positions.
 struct PassGate {
     OpClass cls;
     int k;
+    bool cnot = false;
     int t[2];
     std::complex<double> m[4];
     uint32_t diag_active;
@@ -81,6 +100,11 @@ struct PassGate {
     PassGate(const LoweredGate &g, const std::vector<int> &vpos)
         : cls(g.cls), k(g.k), t{vpos[g.t[0]], g.k > 1 ? vpos[g.t[1]] : 0}, m{g.m[0], g.m[1], g.m[2], g.m[3]},
           diag_active(g.diag_active) {
+        if (cls == OpClass::Dense && k == 2) {
+            cnot = true;
+            if (cnot_target(g) != g.t[0]) std::swap(t[0], t[1]);
+            return;
+        }
         if (k == 2 && t[0] > t[1]) {
             std::swap(t[0], t[1]);
             std::swap(m[1], m[2]);
@@ -299,6 +323,22 @@ template <typename T> PassOp<T> sign_op(const PassGate &d, const std::vector<int
         else if (it != regs.end()) o.b |= 1 << (int)(it - regs.begin());
         else o.pad[nt++] = t;
     }
+    return o;
+}
+
+template <typename T> PassOp<T> cnot_op(const PassGate &g, const std::vector<int> &regs) {
+    constexpr int VB = Traits<T>::VB, S = VB + 6;
+    auto slot = [&](int p) {
+        const auto it = std::find(regs.begin(), regs.end(), p);
+        return it == regs.end() ? -1 : (int)(it - regs.begin());
+    };
+    PassOp<T> o{};
+    o.kind = PO_CNOT;
+    const int t = g.t[0], c = g.t[1];
+    o.b = t < VB ? 2 : (t < S ? 1 : 0);
+    o.a = o.b == 0 ? slot(t) : t - VB;
+    o.active = c < S ? 1u : (slot(c) >= 0 ? 0u : 2u);
+    o.c = o.active == 0 ? slot(c) : c;
     return o;
 }
 
@@ -714,11 +754,17 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
         return SQ_OK;
     }
     const size_t ng = low.size();
-    std::vector<char> mergeable(ng, 0), anywhere(ng, 0);
+    std::vector<char> mergeable(ng, 0);
+    std::vector<uint64_t> need(ng, 0);   // by input qubit
     for (size_t i = 0; i < ng; i++) {
         const LoweredGate &g = low[i];
-        if (g.cls == OpClass::Diag && g.k <= 2) mergeable[i] = anywhere[i] = 1;
-        else if (g.cls == OpClass::Dense && g.k == 1) mergeable[i] = 1;
+        if (g.cls == OpClass::Diag && g.k <= 2) {
+            mergeable[i] = 1;
+        } else if (g.cls == OpClass::Dense) {
+            const int t = g.k == 1 ? g.t[0] : cnot_target(g);
+            mergeable[i] = t >= 0;
+            if (t >= 0) need[i] = 1ULL << t;
+        }
     }
     // the top three lane positions may hold any qubit up to bit 27 of the
     // 16-byte slot index (a lane's offset stays a 32-bit one)
@@ -730,7 +776,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
     key.assign({n, S, kh, moves, std::min(n - 1, 27 + VB), e->plan_beam, (int32_t)ng});
     key.reserve(7 + 5 * ng);
     for (size_t i = 0; i < ng; i++) {
-        key.push_back(mergeable[i] | (anywhere[i] << 1) | (gates[i].nq << 2));
+        key.push_back(mergeable[i] | (gates[i].nq << 2) | (need[i] ? (__builtin_ctzll(need[i]) + 1) << 8 : 0));
         for (int j = 0; j < gates[i].nq && j < 4; j++) key.push_back(gates[i].q[j]);
     }
     const std::vector<sq::SweepStep> *steps_ptr = nullptr;
@@ -742,7 +788,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
     }
     if (!steps_ptr) {
         sq_engine::PlanCacheEntry ent;
-        ent.steps = sq::plan_register_passes(std::vector<sq_gate>(gates, gates + ng), mergeable, anywhere, n, S, kh, moves, std::min(n - 1, 27 + VB),
+        ent.steps = sq::plan_register_passes(std::vector<sq_gate>(gates, gates + ng), mergeable, need, n, S, kh, moves, std::min(n - 1, 27 + VB),
                                              e->plan_beam);
         ent.key = key;
         e->plan_cache.insert(e->plan_cache.begin(), std::move(ent));
@@ -824,7 +870,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
                 const int j = std::min(next[2 * i], next[2 * i + 1]);   // the next gate on either qubit
                 if (j == N) continue;
                 const PassGate &u = lg[j];
-                if (u.cls == OpClass::Dense && folded_from[j] < 0 && !sp[j].ok &&
+                if (u.cls == OpClass::Dense && !u.cnot && folded_from[j] < 0 && !sp[j].ok &&
                     (in_regs(u.t[0]) || (u.t[0] >= VB && u.t[0] < S))) {
                     fold_into[i] = j;
                     folded_from[j] = (int)i;
@@ -866,6 +912,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
                         }
                         continue;
                     }
+                    if (u.cnot && u.t[1] == q) continue;   // a control: phases pass
                     if (sp[j].ok && !zr_done[j]) {
                         f *= sp[j].zr;
                         zr_done[j] = 1;
@@ -919,12 +966,17 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
                 continue;
             }
             if (lg[i].cls == OpClass::Diag) {
-                if (unit_diagonal(lg[i])) {
+                if (tables && unit_diagonal(lg[i])) {
                     run.add(lg[i]);
                     continue;
                 }
             } else if ((run.touched >> lg[i].t[0]) & 1) {
                 settle(i);
+            }
+            if (lg[i].cnot) {
+                if (pend[lg[i].t[0]] != one) flush(i, false);
+                ops.push_back(cnot_op<T>(lg[i], regs));
+                continue;
             }
             PassGate gi = lg[i];
             if (any_split && gi.cls == OpClass::Dense) {
@@ -997,6 +1049,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
         case PO_DIAG_REG2: idx = 6; break;
         case PO_PHASES: idx = 7; oi += o.c; break;   // past its coefficient records
         case PO_DIAG_TAB: idx = o.a < 0 ? 4 : 5; oi += o.c; break;   // past its tables
+        case PO_CNOT: idx = o.b == 2 ? 3 : (o.b == 0 ? 0 : (o.a < 4 ? 1 : 2)); break;
         case PO_ROT_REG: idx = o.c == 1 ? 3 : 0; break;
         case PO_ROT_LANE: idx = o.a < 4 ? 1 : 2; break;
         case PO_SIGN: idx = o.b == 0 ? 4 : (__builtin_popcount((unsigned)o.b) == 1 ? 5 : 6); break;
@@ -1013,7 +1066,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
     }
 
     // upload the program once (in stream order: earlier launches may still read the old one)
-    const size_t need = ops.size() * sizeof(PassOp<T>) + 256;
+    const size_t bytes = ops.size() * sizeof(PassOp<T>) + 256;
     if (dst) {   // caller-owned buffer: never grown
         // (tables can take more records than the gates they stand for)
         if (ops.size() * sizeof(PassOp<T>) > dst_cap && tables)
@@ -1030,14 +1083,14 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
         return SQ_OK;
     }
     if (!ops.empty()) {
-        if (need > e->passprog_cap) {
+        if (bytes > e->passprog_cap) {
             if (hipStreamSynchronize(e->stream) != hipSuccess) return e->fail(SQ_ERR_HIP, "stream sync");
             if (e->d_passprog) (void)hipFree(e->d_passprog);
             e->d_passprog = nullptr;
             e->passprog_cap = 0;
-            hipError_t he = hipMalloc(&e->d_passprog, need * 2);
+            hipError_t he = hipMalloc(&e->d_passprog, bytes * 2);
             if (he != hipSuccess) return e->hip_fail(he, "hipMalloc(pass program)");
-            e->passprog_cap = need * 2;
+            e->passprog_cap = bytes * 2;
         }
         if (int rc = e->upload(e->d_passprog, ops.data(), ops.size() * sizeof(PassOp<T>))) return rc;
     }
@@ -1124,8 +1177,8 @@ int run_plain_t(sq_engine *e, const PlainProgram &prog, const std::vector<Lowere
 
 int sq_engine::build_plain(const sq_gate *gates, const std::vector<LoweredGate> &low, PlainProgram &prog,
                            void *dst, size_t dst_cap) {
-    return dtype == SQ_C128 ? build_plain_t<double>(this, gates, low, prog, dst, dst_cap)
-                            : build_plain_t<float>(this, gates, low, prog, dst, dst_cap);
+    return dtype == SQ_C128 ? build_plain_t<double>(this, gates, low, prog, dst, dst_cap, !keep_order)
+                            : build_plain_t<float>(this, gates, low, prog, dst, dst_cap, !keep_order);
 }
 
 // The second state buffer of the out-of-place permutation pass, allocated
@@ -1149,33 +1202,10 @@ int sq_engine::run_plain_program(const PlainProgram &prog, const std::vector<Low
     return dtype == SQ_C128 ? run_plain_t<double>(this, prog, low) : run_plain_t<float>(this, prog, low);
 }
 
-namespace {
-
-// The target of a U2 whose matrix is exactly a CNOT (control either qubit),
-// or -1.  Local index bit 0 is t[0], bit 1 is t[1].
-int cnot_target(const LoweredGate &g) {
-    if (g.cls != OpClass::Dense || g.k != 2) return -1;
-    const std::complex<double> one(1.0, 0.0), zero(0.0, 0.0);
-    auto is = [&](const int *perm) {   // row r has its one at column perm[r]
-        for (int r = 0; r < 4; r++)
-            for (int c = 0; c < 4; c++)
-                if (g.m[r * 4 + c] != (c == perm[r] ? one : zero)) return false;
-        return true;
-    };
-    static const int flip1[4] = {0, 3, 2, 1};   // control t[0]: bit 1 flips where bit 0 is set
-    static const int flip0[4] = {0, 1, 3, 2};   // control t[1]: bit 0 flips where bit 1 is set
-    if (is(flip1)) return g.t[1];
-    if (is(flip0)) return g.t[0];
-    return -1;
-}
-
-}  // namespace
-
-// Register passes carry one-qubit dense and diagonal gates; a CNOT (written
-// as U2, the reference's way to give one) is H_t CZ H_t with exact 1/sqrt(2)
-// coefficients, so it joins a pass (on complex128 the CZ folds into the
-// second H) instead of taking a pass of its own.  The products differ from
-// the dense 4x4 application by rounding only (|H H - I| = 2^-52).
+// keep_order (complex64 gradients): CNOTs as H_t CZ H_t with exact 1/sqrt(2)
+// coefficients instead of PO_CNOT.  A complex64 gradient carries the rounding
+// of its forward sweep (1e-6) into FP64 results, and callers compare those
+// between versions far more closely; so that sweep rounds as it always has.
 bool sq_engine::expand_cnots(const sq_gate *gates, const std::vector<LoweredGate> &low,
                              std::vector<sq_gate> &g2, std::vector<LoweredGate> &l2) const {
     const int S = (dtype == SQ_C64 ? 1 : 0) + 6;
@@ -1231,7 +1261,7 @@ bool sq_engine::expand_cnots(const sq_gate *gates, const std::vector<LoweredGate
 bool sq_engine::relabel_swaps(const sq_gate *gates, const std::vector<LoweredGate> &low, std::vector<sq_gate> &g2,
                               std::vector<LoweredGate> &l2, std::vector<int> &sigma) const {
     const int S = (dtype == SQ_C64 ? 1 : 0) + 6;
-    if (sweep_mode != 0 || n < S + pass_qbits || lane_moves == 0) return false;   // lane_moves 0: data stays in its lanes
+    if (keep_order || sweep_mode != 0 || n < S + pass_qbits || lane_moves == 0) return false;   // lane_moves 0: data stays in its lanes
     bool any = false;
     for (const auto &g : low) any = any || g.cls == OpClass::Perm;
     if (!any) return false;
@@ -1255,13 +1285,15 @@ bool sq_engine::relabel_swaps(const sq_gate *gates, const std::vector<LoweredGat
 }
 
 int sq_engine::run_plain(const sq_gate *gates, const std::vector<LoweredGate> &low, void *dst, size_t dst_cap) {
-    std::vector<sq_gate> g1, g2;
-    std::vector<LoweredGate> l1, l2;
+    std::vector<sq_gate> g1;
+    std::vector<LoweredGate> l1;
     std::vector<int> sigma;
     const bool sw = relabel_swaps(gates, low, g1, l1, sigma);
     const sq_gate *g = sw ? g1.data() : gates;
     const std::vector<LoweredGate> *l = sw ? &l1 : &low;
-    if (expand_cnots(g, *l, g2, l2)) {
+    std::vector<sq_gate> g2;
+    std::vector<LoweredGate> l2;
+    if (keep_order && expand_cnots(g, *l, g2, l2)) {
         g = g2.data();
         l = &l2;
     }
