@@ -23,6 +23,7 @@
 #include "subquokka_hip.h"
 #include "engine_internal.hpp"
 #include "kernels/adjoint.hpp"
+#include "kernels/hea.hpp"
 #include "kernels/reduce.hpp"
 #include "host/gate_lowering.hpp"
 
@@ -95,8 +96,9 @@ int forward(sq_engine *e, int layers, const double *theta, int ckpt_every, cx<do
     return SQ_OK;
 }
 
+// States of at most one wave row: one launch per gate and per pair of rotations.
 template <typename T>
-int gradient(sq_engine *e, int layers, const double *theta, int ckpt_every, double *energy, double *grad) {
+int gradient_small(sq_engine *e, int layers, const double *theta, int ckpt_every, double *energy, double *grad) {
     const int n = e->n;
     const uint64_t na = e->n_amps();
     const int n_ckpt = (grad && ckpt_every > 0) ? std::max(0, (layers - 1) / ckpt_every) : 0;
@@ -167,6 +169,247 @@ int gradient(sq_engine *e, int layers, const double *theta, int ckpt_every, doub
         grad[p] = s;
     }
     return SQ_OK;
+}
+
+
+// The ansatz as k_hea passes: qubit sets whose bits are resident together --
+// the vector, the lanes and KH register bits first, then KH + 3 qubits at a
+// time (KH in register slots, three in the movable lane positions) -- and, per
+// layer, one pass per set for the rotations and one per set for the ring.
+// The gates keep the list's order: RY on qubit 0, 1, ..., RZ on qubit 0, 1,
+// ... (any position), CNOT 0 -> 1, 1 -> 2, ...; the reverse sweep the opposite.
+struct HeaSet {
+    std::vector<int> qubits;     // ascending
+    std::vector<int> vpos;       // qubit -> virtual position
+    HeaArgs layout{};
+};
+template <typename T> struct HeaPlan {
+    static constexpr int VB = Traits<T>::VB, S = VB + 6;
+    int n, kh;
+    std::vector<HeaSet> sets;
+    HeaPlan(int n_, int kh_) : n(n_), kh(kh_) {
+        for (int q = 0; q < n;) {
+            HeaSet st;
+            const int cnt = std::min(n - q, sets.empty() ? S + kh : kh + kPassLaneHi);
+            for (int i = 0; i < cnt; i++) st.qubits.push_back(q++);
+            std::vector<int> &vpos = st.vpos;
+            vpos.resize(n);
+            for (int i = 0; i < n; i++) vpos[i] = i;
+            std::vector<int> regs;
+            if (sets.empty()) {
+                for (int j = 0; j < kh; j++) regs.push_back(S + j);
+            } else {
+                // the lowest excess qubits take lane positions (runs stay long)
+                const int moved = std::max(0, cnt - kh);
+                for (int i = 0; i < moved; i++) std::swap(vpos[S - kPassLaneHi + i], vpos[st.qubits[i]]);
+                for (int i = moved; i < cnt; i++) regs.push_back(vpos[st.qubits[i]]);
+                for (int p = S; p < n && (int)regs.size() < kh; p++)
+                    if (std::find(regs.begin(), regs.end(), p) == regs.end()) regs.push_back(p);
+                std::sort(regs.begin(), regs.end());
+            }
+            std::vector<int> v2l(n);
+            for (int i = 0; i < n; i++) v2l[vpos[i]] = i;
+            HeaArgs &a = st.layout;
+            a.n_tile_bits = n - S - kh;
+            a.n_tiles = 1ULL << a.n_tile_bits;
+            for (int j = 0; j < kh; j++) { a.hpos[j] = regs[j]; a.reg_pos[j] = v2l[regs[j]]; }
+            for (int k = 0; k < 6; k++) a.lane_pos[k] = v2l[VB + k] - VB;
+            for (int v = S, k = 0; v < n; v++)
+                if (std::find(regs.begin(), regs.end(), v) == regs.end()) a.tile_pos[k++] = v2l[v];
+            sets.push_back(std::move(st));
+        }
+    }
+    // a lane's offset holds slot bits up to kPassMaxSlotBit
+    bool fits() const {
+        for (const auto &st : sets)
+            for (int k = 0; k < 6; k++) if (st.layout.lane_pos[k] < 0 || st.layout.lane_pos[k] > kPassMaxSlotBit) return false;
+        return n - S - kh <= kPassMaxTileBits;
+    }
+    void where(const HeaSet &st, int q, int32_t &w, int32_t &at) const {
+        const int v = st.vpos[q];
+        const int *e = st.layout.hpos + kh, *it = std::find(st.layout.hpos, e, v);
+        w = it != e ? HW_SLOT : (v < VB ? HW_VEC : (v < S ? HW_LANE : HW_TILE));
+        at = it != e ? (int32_t)(it - st.layout.hpos) : v;
+    }
+    HeaOp target(const HeaSet &st, int kind, int q) const {   // a gate whose qubit is resident
+        HeaOp o{};
+        o.kind = kind;
+        where(st, q, o.where, o.at);
+        if (o.where == HW_LANE) o.at -= VB;
+        return o;
+    }
+    HeaOp cnot(const HeaSet &st, int c, int t) const {
+        HeaOp o = target(st, HO_CNOT, t);
+        where(st, c, o.cwhere, o.cat);
+        return o;
+    }
+};
+struct HeaPass {
+    size_t set, op_begin, n_ops;
+    std::vector<int> slots;   // partial slots of its accumulators
+    int restore = -1;         // checkpoint to re-anchor psi to before the pass
+    int save = -1;            // checkpoint to take after the pass
+};
+
+template <typename T, int NV>
+int launch_hea(sq_engine *e, int kh, const HeaArgs &a, unsigned grid) {
+    cx<T> *psi = reinterpret_cast<cx<T> *>(e->d_state), *lam = reinterpret_cast<cx<T> *>(e->d_aux);
+    const size_t lds = (size_t)a.n_acc * kBlock * sizeof(double);
+    switch (kh) {
+    case 1: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hea<T, 1, NV>), grid, kBlock, lds, e->stream, psi, lam, a); break;
+    case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hea<T, 2, NV>), grid, kBlock, lds, e->stream, psi, lam, a); break;
+    case 3: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hea<T, 3, NV>), grid, kBlock, lds, e->stream, psi, lam, a); break;
+    case 4: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hea<T, 4, NV>), grid, kBlock, lds, e->stream, psi, lam, a); break;
+    default:
+        if constexpr (NV == 1) { hipLaunchKernelGGL(HIP_KERNEL_NAME(k_hea<T, 5, NV>), grid, kBlock, lds, e->stream, psi, lam, a); break; }
+        return e->fail(SQ_ERR_ARG, "internal: bad pass width");
+    }
+    return e->check_launch("k_hea");
+}
+
+template <typename T>
+int gradient(sq_engine *e, int layers, const double *theta, int ckpt_every, double *energy, double *grad) {
+    constexpr int VB = Traits<T>::VB, S = VB + 6;
+    const int n = e->n;
+    // register bits: as many as leave about 1024 waves, two at least; both
+    // vectors of the reverse sweep: four (16 x 2 vectors a lane)
+    const int most = n - S;
+    if (most < 1) return gradient_small<T>(e, layers, theta, ckpt_every, energy, grad);
+    const HeaPlan<T> fwd(n, std::min(most, std::max(2, std::min(5, most - 10))));
+    const HeaPlan<T> rev(n, std::min(most, std::max(2, std::min(4, most - 10))));
+    if (!fwd.fits() || !rev.fits()) return gradient_small<T>(e, layers, theta, ckpt_every, energy, grad);
+    const uint64_t na = e->n_amps();
+    const int n_ckpt = (grad && ckpt_every > 0) ? std::max(0, (layers - 1) / ckpt_every) : 0;
+    const size_t n_params = (size_t)2 * n * layers;
+    std::vector<HeaOp> ops;
+    std::vector<HeaPass> up, down;
+    auto open = [&](std::vector<HeaPass> &list, size_t set) { list.push_back({set, ops.size(), 0, {}}); };
+    auto close = [&](std::vector<HeaPass> &list) {
+        list.back().n_ops = ops.size() - list.back().op_begin;
+        if (!list.back().n_ops) list.pop_back();
+    };
+    for (int l = 0; l < layers; l++) {
+        const double *ty = theta + (size_t)l * 2 * n, *tz = ty + n;
+        for (size_t k = 0; k < fwd.sets.size(); k++) {
+            const HeaSet &st = fwd.sets[k];
+            open(up, k);
+            for (int q : st.qubits) {
+                HeaOp o = fwd.target(st, HO_RY, q);
+                o.c = std::cos(ty[q] / 2);
+                o.s = std::sin(ty[q] / 2);
+                ops.push_back(o);
+            }
+            for (int q = 0; k + 1 == fwd.sets.size() && q < n; q++) {   // after every RY: diagonal, any position
+                HeaOp o{};
+                o.kind = HO_RZ;
+                fwd.where(st, q, o.where, o.at);
+                o.c = std::cos(tz[q] / 2);
+                o.s = std::sin(tz[q] / 2);
+                ops.push_back(o);
+            }
+            close(up);
+        }
+        for (size_t k = 0; n > 1 && k < fwd.sets.size(); k++) {
+            const HeaSet &st = fwd.sets[k];
+            open(up, k);
+            for (int t : st.qubits) if (t > 0) ops.push_back(fwd.cnot(st, t - 1, t));
+            if (k + 1 == fwd.sets.size()) ops.push_back(fwd.cnot(st, n - 1, 0));   // bit 0 is resident in every set
+            close(up);
+        }
+        if (n_ckpt && (l + 1) % ckpt_every == 0 && l + 1 < layers) up.back().save = (l + 1) / ckpt_every - 1;
+    }
+    for (int l = layers - 1; grad && l >= 0; l--) {
+        const double *ty = theta + (size_t)l * 2 * n, *tz = ty + n;
+        const size_t first = down.size();
+        for (size_t k = rev.sets.size(); n > 1 && k-- > 0;) {
+            const HeaSet &st = rev.sets[k];
+            open(down, k);
+            if (k + 1 == rev.sets.size()) ops.push_back(rev.cnot(st, n - 1, 0));
+            for (size_t i = st.qubits.size(); i-- > 0;)
+                if (st.qubits[i] > 0) ops.push_back(rev.cnot(st, st.qubits[i] - 1, st.qubits[i]));
+            close(down);
+        }
+        for (size_t k = rev.sets.size(); k-- > 0;) {
+            const HeaSet &st = rev.sets[k];
+            open(down, k);
+            for (size_t i = st.qubits.size(); i-- > 0;) {
+                const int q = st.qubits[i];
+                HeaOp o = rev.target(st, HO_ROT2, q);
+                o.c = std::cos(ty[q] / 2);
+                o.s = std::sin(ty[q] / 2);
+                o.cz = std::cos(tz[q] / 2);
+                o.sz = std::sin(tz[q] / 2);
+                o.acc = (int32_t)down.back().slots.size();
+                down.back().slots.push_back(l * 2 * n + q);
+                down.back().slots.push_back(l * 2 * n + n + q);
+                ops.push_back(o);
+            }
+            close(down);
+        }
+        if (n_ckpt && (l + 1) % ckpt_every == 0 && l + 1 < layers) down[first].restore = (l + 1) / ckpt_every - 1;
+    }
+    // buffers: partials [slot][block], their sums, the program
+    const unsigned red_grid = (unsigned)std::min<uint64_t>(kRedBlocks, std::max<uint64_t>(1, rev.sets[0].layout.n_tiles * 64 / kBlock));
+    const size_t part_bytes = grad ? n_params * red_grid * sizeof(double) : 0;
+    const size_t out_bytes = (n_params * sizeof(double) + 255) / 256 * 256;
+    const size_t prog_at = (part_bytes + out_bytes + 255) / 256 * 256;
+    int rc = ensure(e, &e->d_gradpart, &e->gradpart_cap, prog_at + ops.size() * sizeof(HeaOp) + 256, "hipMalloc(gradient partials)");
+    if (!rc && grad) rc = ensure(e, &e->d_aux, &e->aux_cap, e->state_bytes(), "hipMalloc(lambda)");
+    if (!rc && n_ckpt)
+        rc = ensure(e, &e->d_ckpt, &e->ckpt_cap, (size_t)n_ckpt * na * sizeof(cx<double>), "hipMalloc(checkpoints)");
+    if (rc) return rc;
+    double *part = static_cast<double *>(e->d_gradpart);
+    double *d_out = reinterpret_cast<double *>(static_cast<char *>(e->d_gradpart) + part_bytes);
+    const HeaOp *d_ops = reinterpret_cast<const HeaOp *>(static_cast<char *>(e->d_gradpart) + prog_at);
+    cx<double> *ckpt = n_ckpt ? static_cast<cx<double> *>(e->d_ckpt) : nullptr;
+    if ((rc = e->upload(const_cast<HeaOp *>(d_ops), ops.data(), ops.size() * sizeof(HeaOp)))) return rc;
+    if ((rc = sq_init_zero(e))) return rc;
+    cx<T> *psi = reinterpret_cast<cx<T> *>(e->d_state), *lam = reinterpret_cast<cx<T> *>(e->d_aux);
+    for (const HeaPass &p : up) {
+        HeaArgs a = fwd.sets[p.set].layout;
+        a.ops = d_ops + p.op_begin;
+        a.n_ops = (int)p.n_ops;
+        const int slot = e->stat_begin("hea_fwd", 2.0 * e->amp_bytes() * (double)na);
+        rc = launch_hea<T, 1>(e, fwd.kh, a, e->grid_flat(a.n_tiles, kBlock / 64));
+        e->stat_end(slot);
+        if (rc) return rc;
+        if (p.save >= 0) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_convert<T, double>), e->grid_for(na, kBlock), kBlock, 0, e->stream,
+                               psi, ckpt + (size_t)p.save * na, na);
+            if ((rc = e->check_launch("checkpoint"))) return rc;
+        }
+    }
+    double v[2];
+    if ((rc = e->norm_zz(v))) return rc;
+    if (energy) *energy = v[1];
+    if (!grad) return SQ_OK;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_apply_zz_ring<T>), e->grid_for(na, kBlock), kBlock, 0, e->stream, psi, lam, na, n);
+    if ((rc = e->check_launch("k_apply_zz_ring"))) return rc;
+    for (const HeaPass &p : down) {
+        if (p.restore >= 0) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_convert<double, T>), e->grid_for(na, kBlock), kBlock, 0, e->stream,
+                               ckpt + (size_t)p.restore * na, psi, na);
+            if ((rc = e->check_launch("re-anchor"))) return rc;
+        }
+        HeaArgs a = rev.sets[p.set].layout;
+        a.ops = d_ops + p.op_begin;
+        a.n_ops = (int)p.n_ops;
+        a.n_acc = (int)p.slots.size();
+        if (a.n_acc > kHeaMaxAcc) return e->fail(SQ_ERR_ARG, "internal: too many terms in a pass");
+        std::copy(p.slots.begin(), p.slots.end(), a.slot);
+        a.part = part;
+        const int slot = e->stat_begin(a.n_acc ? "hea_terms" : "hea_ring2", 4.0 * e->amp_bytes() * (double)na);
+        rc = launch_hea<T, 2>(e, rev.kh, a, a.n_acc ? red_grid : e->grid_flat(a.n_tiles, kBlock / 64));
+        e->stat_end(slot);
+        if (rc) return rc;
+    }
+    if (!n_params) return SQ_OK;
+    hipLaunchKernelGGL(k_sum_slots, (unsigned)((n_params + kBlock / 64 - 1) / (kBlock / 64)), kBlock, 0, e->stream,
+                       (const double *)part, (uint64_t)red_grid, (int)n_params, d_out);
+    if ((rc = e->check_launch("k_sum_slots"))) return rc;
+    hipError_t he = hipMemcpyAsync(grad, d_out, n_params * sizeof(double), hipMemcpyDeviceToHost, e->stream);
+    if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
+    return he == hipSuccess ? SQ_OK : e->hip_fail(he, "gradient sums");
 }
 
 }  // namespace
