@@ -166,7 +166,9 @@ int sq_apply_fused(sq_engine *e, const sq_fused *blocks, uint64_t n);
 /* Fused blocks from gates: block i is block_sizes[i] consecutive gates acting on
  * at most five qubits (the planner's mode 1 output).  Each block is composed in
  * FP64 on the GPU, then applied on MFMA (FP32 accumulation for SQ_C64, FP64 for
- * SQ_C128).  The result equals applying the gates in order. */
+ * SQ_C128).  The result equals applying the gates in order; SQ_C128 blocks of
+ * one-qubit, diagonal, SWAP and CNOT gates on 25 qubits and more are applied as
+ * that list, in register passes (sweep_mode 0), which reads the state fewer times. */
 int sq_run_fused(sq_engine *e, const sq_gate *gates, const uint32_t *block_sizes, uint64_t n_blocks);
 /* A plain gate list (the sq_apply_gates / MEM_Runner::run(vector<Gate*>&) input,
  * MEM_Runner.cpp:101-134) as fused passes on a complex64 state: the engine cuts

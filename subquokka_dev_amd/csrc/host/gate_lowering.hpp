@@ -178,6 +178,24 @@ inline int lower_gate(const sq_gate &g, int n_qubits, LoweredGate &out, std::str
     return SQ_OK;
 }
 
+// The target of a U2 whose matrix is exactly a CNOT (control either qubit; the
+// reference's way to write one), or -1.  Local index bit 0 is t[0], bit 1 is t[1].
+inline int cnot_target(const LoweredGate &g) {
+    if (g.cls != OpClass::Dense || g.k != 2) return -1;
+    const std::complex<double> one(1.0, 0.0), zero(0.0, 0.0);
+    auto is = [&](const int *perm) {   // row r has its one at column perm[r]
+        for (int r = 0; r < 4; r++)
+            for (int c = 0; c < 4; c++)
+                if (g.m[r * 4 + c] != (c == perm[r] ? one : zero)) return false;
+        return true;
+    };
+    static const int flip1[4] = {0, 3, 2, 1};   // control t[0]: bit 1 flips where bit 0 is set
+    static const int flip0[4] = {0, 1, 3, 2};   // control t[1]: bit 0 flips where bit 1 is set
+    if (is(flip1)) return g.t[1];
+    if (is(flip0)) return g.t[0];
+    return -1;
+}
+
 // The gate with its targets mapped through sigma (a permutation of qubits:
 // the layout after VSWAP data moves, or a pass's virtual positions).  A two-qubit gate keeps its internal basis
 // (local bit j <-> j-th smallest target), so when the mapping reverses the

@@ -196,6 +196,29 @@ int build_program(sq_engine *e, const sq_gate *gates, const uint32_t *sizes, uin
     return SQ_OK;
 }
 
+// Lowers a block list into the engine's workspace with build_program's checks;
+// carried: the register passes run every gate of it.
+int check_blocks(sq_engine *e, const sq_gate *gates, const uint32_t *sizes, uint64_t n_blocks, bool &carried) {
+    e->ws_low.clear();
+    size_t first = 0;
+    for (uint64_t b = 0; b < n_blocks; b++) {
+        uint64_t used = 0;
+        for (uint32_t i = 0; i < sizes[b]; i++) {
+            const sq_gate &g = gates[first + i];
+            e->ws_low.emplace_back();
+            LoweredGate &lg = e->ws_low.back();
+            int rc = e->lower(g, lg);
+            if (rc) { e->err += " (gate " + std::to_string(first + i) + ")"; return rc; }
+            for (int j = 0; j < g.nq; j++) used |= 1ULL << g.q[j];
+            carried = carried && (lg.cls != OpClass::Dense || lg.k == 1 || sq::cnot_target(lg) >= 0);
+        }
+        if (__builtin_popcountll(used) > kFusedK)
+            return e->fail(SQ_ERR_ARG, "block " + std::to_string(b) + " acts on more than 5 qubits");
+        first += sizes[b];
+    }
+    return SQ_OK;
+}
+
 // ---------------------------------------------------------------------------
 // Fused passes (complex64): the plain gate list cut into passes over tiles of
 // r qubits, each pass's gates grouped into four-qubit blocks (kernels/fpass.hpp).
@@ -437,6 +460,24 @@ extern "C" int sq_run_fused(sq_engine *e, const sq_gate *gates, const uint32_t *
     if (e->n < kFusedK) return e->fail(SQ_ERR_ARG, "fused blocks need at least 5 qubits");
     if (hipSetDevice(e->device) != hipSuccess) return SQ_ERR_HIP;
     FusedProgram p;
+    // Large complex128 states: blocks whose gates the register passes carry run
+    // as the list they are -- one read and write of the state per pass of about
+    // 50 gates instead of one per block of about 12, and no composition (25
+    // qubits, 300 gates in 25 blocks: 5.53 -> 2.10 ms).  FP64 matrix
+    // instructions have the vector rate here, and a 32x32 block spends 256 of
+    // its products per amplitude.  The passes' schedule takes about 1.5 ms on the
+    // first call with a new structure (first call, 20 qubits: 0.47 ms with blocks,
+    // 1.5 ms with passes; 24 qubits x 2 layers: 1.4 and 1.8 ms; 25 qubits: 6.0
+    // and 4.6 ms), so smaller states keep the blocks; so do complex64 ones, whose products are composed in FP64.
+    constexpr int kPassesFromQubits = 25;
+    if (e->dtype == SQ_C128 && e->sweep_mode == 0 && e->n >= kPassesFromQubits) {
+        uint64_t total = 0;
+        for (uint64_t b = 0; b < n_blocks; b++) total += block_sizes[b];
+        bool carried = true;
+        int rc = check_blocks(e, gates, block_sizes, n_blocks, carried);
+        if (rc) return rc;
+        if (carried) return e->apply_plain(gates, total, e->ws_low);
+    }
     int rc = build_program(e, gates, block_sizes, n_blocks, kFusedK, nullptr, p);
     if (rc) return rc;
     cx<double> *u = nullptr;

@@ -69,24 +69,6 @@ private:
     }
 };
 
-// The target of a U2 whose matrix is exactly a CNOT (control either qubit; the
-// reference's way to write one), or -1.  Local index bit 0 is t[0], bit 1 is t[1].
-int cnot_target(const LoweredGate &g) {
-    if (g.cls != OpClass::Dense || g.k != 2) return -1;
-    const std::complex<double> one(1.0, 0.0), zero(0.0, 0.0);
-    auto is = [&](const int *perm) {   // row r has its one at column perm[r]
-        for (int r = 0; r < 4; r++)
-            for (int c = 0; c < 4; c++)
-                if (g.m[r * 4 + c] != (c == perm[r] ? one : zero)) return false;
-        return true;
-    };
-    static const int flip1[4] = {0, 3, 2, 1};   // control t[0]: bit 1 flips where bit 0 is set
-    static const int flip0[4] = {0, 1, 3, 2};   // control t[1]: bit 0 flips where bit 1 is set
-    if (is(flip1)) return g.t[1];
-    if (is(flip0)) return g.t[0];
-    return -1;
-}
-
 // A gate of a register pass: dense on one qubit, diagonal on one or two (t
 // ascending) or a CNOT (t: target, control), in the pass's virtual positions.
 struct PassGate {
@@ -102,7 +84,7 @@ struct PassGate {
           diag_active(g.diag_active) {
         if (cls == OpClass::Dense && k == 2) {
             cnot = true;
-            if (cnot_target(g) != g.t[0]) std::swap(t[0], t[1]);
+            if (sq::cnot_target(g) != g.t[0]) std::swap(t[0], t[1]);
             return;
         }
         if (k == 2 && t[0] > t[1]) {
@@ -761,7 +743,7 @@ int build_plain_t(sq_engine *e, const sq_gate *gates, const std::vector<LoweredG
         if (g.cls == OpClass::Diag && g.k <= 2) {
             mergeable[i] = 1;
         } else if (g.cls == OpClass::Dense) {
-            const int t = g.k == 1 ? g.t[0] : cnot_target(g);
+            const int t = g.k == 1 ? g.t[0] : sq::cnot_target(g);
             mergeable[i] = t >= 0;
             if (t >= 0) need[i] = 1ULL << t;
         }
@@ -1211,13 +1193,13 @@ bool sq_engine::expand_cnots(const sq_gate *gates, const std::vector<LoweredGate
     const int S = (dtype == SQ_C64 ? 1 : 0) + 6;
     if (sweep_mode != 0 || n < S + pass_qbits) return false;   // no register passes
     bool any = false;
-    for (const auto &g : low) any = any || cnot_target(g) >= 0;
+    for (const auto &g : low) any = any || sq::cnot_target(g) >= 0;
     if (!any) return false;
     const double s = 0.70710678118654752440;
     g2.clear();
     l2.clear();
     for (size_t i = 0; i < low.size(); i++) {
-        const int t = cnot_target(low[i]);
+        const int t = sq::cnot_target(low[i]);
         if (t < 0) {
             g2.push_back(gates[i]);
             l2.push_back(low[i]);
