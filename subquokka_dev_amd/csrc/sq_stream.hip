@@ -447,11 +447,16 @@ int sq_engine::stream_apply(const std::vector<sq_gate> &gates, const std::vector
         }
         // the pass's gates as register passes over a W-qubit group: planned and
         // uploaded once, run on every group
+        // Waits around the program's copy: without them the host queues the next
+        // passes' transfers ahead, which is slower (24 qubits, groups of 2^20
+        // amplitudes, 117-120 ms without in three runs, 82-93 ms with in four).
         PlainProgram prog;
+        if (hipStreamSynchronize(stream) != hipSuccess) { rc = fail(SQ_ERR_HIP, "stream sync"); break; }
         n = W;
         rc = build_plain(pgates.data(), pg, prog);
         n = saved_n;
         if (rc) break;
+        if (hipStreamSynchronize(stream) != hipSuccess) { rc = fail(SQ_ERR_HIP, "stream sync"); break; }
         std::vector<uint64_t> run_off(1ULL << h), run_off_bytes(1ULL << h);   // host offset of run r within a group
         for (uint64_t r = 0; r < run_off.size(); r++) {
             uint64_t o = 0;
