@@ -548,7 +548,10 @@ int adjoint_general(sq_engine *e, const sq_gate *gates, const int32_t *param, ui
     // complex64: each gate is un-applied and its term taken where the list has
     // it, so that the FP32 rounding, and with it the gradient to all digits,
     // stays what it is (see keep_order)
-    const bool runs = tiles && sizeof(T) == 8;
+    // Without register passes too (complex128: under 11 qubits): a run's gates would
+    // be one launch each to un-apply, after the launch that takes the terms (MaxCut
+    // gradient, 9 qubits, five layers: 2.54 ms as runs, 2.09 ms gate by gate).
+    const bool runs = tiles && sizeof(T) == 8 && e->sweep_mode == 0 && n >= Traits<T>::VB + 6 + e->pass_qbits;
     struct KeepOrder {
         sq_engine *e;
         KeepOrder(sq_engine *x, bool on) : e(x) { e->keep_order = on; }
